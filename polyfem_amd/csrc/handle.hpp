@@ -127,6 +127,8 @@ void plain_energy(Handle &h, const double *x, double *energy, double *per_elemen
 void energy_into(Handle &h, const double *x, double *energy, double *partial, double *part);
 void plain_gradient(Handle &h, const double *x, double *g, double *energy);
 void plain_hessian(Handle &h, const double *x, void *values, bool project_to_psd = false);
+// element Hessians of SaintVenant, FixedCorotational and MooneyRivlin in the block tiles (points.hip)
+void points_hessian(Handle &h, const double *x, void *hloc);
 // every element's local Hessian in the block tiles projected onto the PSD cone (psd.hip)
 void psd_project_blocks(Handle &h, void *hloc);
 void plain_hvp(Handle &h, const double *x, const double *v, double *y);

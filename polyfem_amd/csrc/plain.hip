@@ -222,6 +222,7 @@ __global__ __launch_bounds__(64) void k_grad_factors(DevMesh<T> m, const double 
 }
 
 // Upper-triangle local Hessian blocks (a <= b, s(a,b) = a NB - a(a-1)/2 + b - a)
+// of NeoHookean and linear elasticity (points.hip has the other materials)
 // in tiles of 64 elements: block s of element e is the 9 values at
 // hloc[(((e / 64) NBLK + s) 64 + e % 64) 9], row-major.  A wavefront computes
 // the blocks of its 64 elements and writes each block index s as one
@@ -242,49 +243,25 @@ __global__ __launch_bounds__(HB) void k_hessian(DevMesh<T> m, const double *__re
     Elem<T, ORDER, NQ> el;
     load_geometry(m, ee, el);
     if (MAT != MAT_LE) gather(m, ee, x, el.U);
-    // the weight of the rules that weigh every point alike (isotropic term)
-    const T w0 = el.det * T(quad_weight(NQ, 0));
     // per point: M = F^{-T} J^{-T} (k_a = M RG(q,a)) and the two curvature
     // weights; the k vectors are formed per block row and column to keep the
-    // register footprint small.  SaintVenant adds the S-weighted metric and
-    // mu F F^T per point.
-    // FixedCorotational adds the rotation R and K^{-1} per point.
-    constexpr int NX = MAT == MAT_SV || MAT == MAT_FC ? NQ : 1;
-    // MooneyRivlin forms its blocks from the directional stress derivative
-    // (below) and keeps nothing per point
-    constexpr int NM = MAT == MAT_MR ? 1 : NQ;
-    T Mq[NM][9], cl[NM], cc[NM], sg6[NX][6], ff6[NX][9];
+    // register footprint small
+    T Mq[NQ][9], cl[NQ], cc[NQ];
 #pragma unroll
-    for (int q = 0; q < NM; ++q) {
+    for (int q = 0; q < NQ; ++q) {
         const T w = el.det * T(quad_weight(NQ, q));
-        if constexpr (MAT == MAT_MR) {
-#pragma unroll
-            for (int i = 0; i < 9; ++i) Mq[q][i] = T(0);
-            cl[q] = cc[q] = T(0);
-            continue;
-        }
         Kin<T> k;
         if (MAT != MAT_LE) field_grad<T, ORDER, NQ>(q, el.U, el.jit, k.H);
-        if (MAT == MAT_NH || MAT == MAT_FC) kinematics(k);
+        if (MAT == MAT_NH) kinematics(k);
         hess_qp<T, MAT>(k, el.jit, el.lam, el.mu, w, Mq[q], cl[q], cc[q]);
-        if constexpr (MAT == MAT_SV) sv_extra(k.H, el.jit, el.lam, el.mu, w, sg6[q], ff6[q]);
-        if constexpr (MAT == MAT_FC) {
-            // sg6: K^{-1}; ff6: the rows of R
-            FcKin<T> f;
-            fc_kinematics(k.H, f);
-#pragma unroll
-            for (int i = 0; i < 6; ++i) sg6[q][i] = f.Ki6[i];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) ff6[q][i] = f.Q[i] + (i % 4 == 0 ? T(1) : T(0));
-        }
     }
     T g6[6];
     metric(el.jit, g6);
-    const T cm = (MAT == MAT_FC ? T(2) : T(1)) * w0 * el.mu;
+    const T cm = el.det * T(quad_weight(NQ, 0)) * el.mu;
     T *st = stage[wv];
     T *out = hloc + tile * NBLK * 576;
     const RefTab<T, ORDER, NQ> &tb = ref_tab<T, ORDER, NQ>();
-    // the isotropic term sum_q w_q cm' RG(q,a)^T G RG(q,b): from the summed
+    // the isotropic term sum_q w_q mu RG(q,a)^T G RG(q,b): from the summed
     // table for the rules that weigh every point alike, point by point otherwise
     auto iso = [&](int a, int b, const T *c) {
         if constexpr (quad_uniform(NQ)) {
@@ -294,7 +271,7 @@ __global__ __launch_bounds__(HB) void k_hessian(DevMesh<T> m, const double *__re
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 const T *ra = tb.rg + (q * NB + a) * 3, *rb = tb.rg + (q * NB + b) * 3;
-                s += (MAT == MAT_FC ? T(2) : T(1)) * el.det * T(quad_weight(NQ, q)) * el.mu * sym_form(ra, g6, rb);
+                s += el.det * T(quad_weight(NQ, q)) * el.mu * sym_form(ra, g6, rb);
             }
             return s;
         }
@@ -302,9 +279,9 @@ __global__ __launch_bounds__(HB) void k_hessian(DevMesh<T> m, const double *__re
     // a and b are uniform over the wavefront: the table reads are scalar
 #pragma unroll 1
     for (int a = 0; a < NB; ++a) {
-        T Ka[NM][3];
+        T Ka[NQ][3];
 #pragma unroll
-        for (int q = 0; q < NM; ++q)
+        for (int q = 0; q < NQ; ++q)
 #pragma unroll
             for (int mm = 0; mm < 3; ++mm) {
                 const T *r = tb.rg + (q * NB + a) * 3;
@@ -313,102 +290,23 @@ __global__ __launch_bounds__(HB) void k_hessian(DevMesh<T> m, const double *__re
         // not unrolled: the k_b of all columns at once would not fit in registers
 #pragma unroll 1
         for (int b = a; b < NB; ++b) {
-            T Kb[NM][3];
+            T Kb[NQ][3];
 #pragma unroll
-            for (int q = 0; q < NM; ++q)
+            for (int q = 0; q < NQ; ++q)
 #pragma unroll
                 for (int mm = 0; mm < 3; ++mm) {
                     const T *r = tb.rg + (q * NB + b) * 3;
                     Kb[q][mm] = Mq[q][mm * 3] * r[0] + Mq[q][mm * 3 + 1] * r[1] + Mq[q][mm * 3 + 2] * r[2];
                 }
             const int s = a * NB - a * (a - 1) / 2 + (b - a);
-            const T *c = tb.rgg + (a * NB + b) * 6;
-            T gd = T(0), xf[6] = {T(0), T(0), T(0), T(0), T(0), T(0)};
-            T xr[9] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};
-            if constexpr (MAT == MAT_FC) {
-                // -2 mu da sum_q (G_a x r_m)^T K^{-1} (G_b x r_n), r_m the rows of R
-                gd = iso(a, b, c);
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    const T w = el.det * T(quad_weight(NQ, q));
-                    const T *ra = tb.rg + (q * NB + a) * 3, *rb = tb.rg + (q * NB + b) * 3;
-                    T Ga[3], Gb[3];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        Ga[i] = ra[0] * el.jit[0 * 3 + i] + ra[1] * el.jit[1 * 3 + i] + ra[2] * el.jit[2 * 3 + i];
-                        Gb[i] = rb[0] * el.jit[0 * 3 + i] + rb[1] * el.jit[1 * 3 + i] + rb[2] * el.jit[2 * 3 + i];
-                    }
-                    const T *R = ff6[q], *Ki = sg6[q];
-                    T ca[3][3], kb[3][3];
-#pragma unroll
-                    for (int mm = 0; mm < 3; ++mm) {
-                        const T *r = R + mm * 3;
-                        ca[mm][0] = Ga[1] * r[2] - Ga[2] * r[1];
-                        ca[mm][1] = Ga[2] * r[0] - Ga[0] * r[2];
-                        ca[mm][2] = Ga[0] * r[1] - Ga[1] * r[0];
-                        const T cb0 = Gb[1] * r[2] - Gb[2] * r[1], cb1 = Gb[2] * r[0] - Gb[0] * r[2],
-                                cb2 = Gb[0] * r[1] - Gb[1] * r[0];
-                        kb[mm][0] = Ki[0] * cb0 + Ki[3] * cb1 + Ki[4] * cb2;
-                        kb[mm][1] = Ki[3] * cb0 + Ki[1] * cb1 + Ki[5] * cb2;
-                        kb[mm][2] = Ki[4] * cb0 + Ki[5] * cb1 + Ki[2] * cb2;
-                    }
-                    const T cr = -T(2) * el.mu * w;
-#pragma unroll
-                    for (int mm = 0; mm < 3; ++mm)
-#pragma unroll
-                        for (int nn = 0; nn < 3; ++nn)
-                            xr[mm * 3 + nn] += cr * (ca[mm][0] * kb[nn][0] + ca[mm][1] * kb[nn][1] + ca[mm][2] * kb[nn][2]);
-                }
-            } else if constexpr (MAT == MAT_MR) {
-                // column n of the block: sum_q da dP[e_n G_b^T] G_a (the
-                // kinematics of each point are formed again per block)
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    const T w = el.det * T(quad_weight(NQ, q));
-                    Kin<T> k;
-                    field_grad<T, ORDER, NQ>(q, el.U, el.jit, k.H);
-                    kinematics(k);
-                    const T *ra = tb.rg + (q * NB + a) * 3, *rb = tb.rg + (q * NB + b) * 3;
-                    T Ga[3], Gb[3];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        Ga[i] = ra[0] * el.jit[0 * 3 + i] + ra[1] * el.jit[1 * 3 + i] + ra[2] * el.jit[2 * 3 + i];
-                        Gb[i] = rb[0] * el.jit[0 * 3 + i] + rb[1] * el.jit[1 * 3 + i] + rb[2] * el.jit[2 * 3 + i];
-                    }
-#pragma unroll
-                    for (int nn = 0; nn < 3; ++nn) {
-                        T W[9], dP[9];
-#pragma unroll
-                        for (int i = 0; i < 9; ++i) W[i] = i / 3 == nn ? Gb[i % 3] : T(0);
-                        mr_dstress(k, el.lam, el.mu, el.p3, W, dP);
-#pragma unroll
-                        for (int mm = 0; mm < 3; ++mm)
-                            xr[mm * 3 + nn] += w * (dP[mm * 3] * Ga[0] + dP[mm * 3 + 1] * Ga[1] + dP[mm * 3 + 2] * Ga[2]);
-                    }
-                }
-            } else if constexpr (MAT == MAT_SV) {
-                // sum_q [ (G_a^T S G_b) I + mu (G_a . G_b) F F^T ] da
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    const T *ra = tb.rg + (q * NB + a) * 3, *rb = tb.rg + (q * NB + b) * 3;
-                    gd += sym_form(ra, sg6[q], rb);
-                    const T gq = sym_form(ra, g6, rb);
-#pragma unroll
-                    for (int i = 0; i < 6; ++i) xf[i] += gq * ff6[q][i];
-                }
-            } else {
-                gd = iso(a, b, c);
-            }
-            const int sym[9] = {0, 3, 4, 3, 1, 5, 4, 5, 2};
+            const T gd = iso(a, b, tb.rgg + (a * NB + b) * 6);
 #pragma unroll
             for (int mm = 0; mm < 3; ++mm)
 #pragma unroll
                 for (int nn = 0; nn < 3; ++nn) {
                     T v = mm == nn ? gd : T(0);
-                    if constexpr (MAT == MAT_SV) v += xf[sym[mm * 3 + nn]];
-                    if constexpr (MAT == MAT_FC || MAT == MAT_MR) v += xr[mm * 3 + nn];
 #pragma unroll
-                    for (int q = 0; q < NM; ++q) v += cl[q] * Ka[q][mm] * Kb[q][nn] + cc[q] * Kb[q][mm] * Ka[q][nn];
+                    for (int q = 0; q < NQ; ++q) v += cl[q] * Ka[q][mm] * Kb[q][nn] + cc[q] * Kb[q][mm] * Ka[q][nn];
                     st[lane * 9 + mm * 3 + nn] = v;
                 }
             // the wavefront's 64 blocks s are 576 consecutive values
@@ -1922,16 +1820,20 @@ void plain_hessian(Handle &h, const double *x, void *values, bool project_to_psd
     const GatherPlan &p = h.blk_plan;
     h.hloc.reserve(h.value_size() * size_t((h.n_elements + 63) / 64) * 64 * h.n_blocks_sym() * 9);
     dispatch(h, [&]<typename T, int O, int Q, int M>() {
-        auto hess = [&]<int HB>() {
-            k_hessian<T, O, Q, M, HB><<<grid_for(h.n_elements, HB), HB, 0, h.stream>>>(h.mesh<T>(), x, h.hloc.as<T>());
-        };
-        if (h.tune_hessian_threads == 64)
-            hess.template operator()<64>();
-        else if (h.tune_hessian_threads == 128)
-            hess.template operator()<128>();
-        else
-            hess.template operator()<256>();
-        PF_LAUNCH_CHECK();
+        if constexpr (M == MAT_NH || M == MAT_LE) {
+            auto hess = [&]<int HB>() {
+                k_hessian<T, O, Q, M, HB><<<grid_for(h.n_elements, HB), HB, 0, h.stream>>>(h.mesh<T>(), x, h.hloc.as<T>());
+            };
+            if (h.tune_hessian_threads == 64)
+                hess.template operator()<64>();
+            else if (h.tune_hessian_threads == 128)
+                hess.template operator()<128>();
+            else
+                hess.template operator()<256>();
+            PF_LAUNCH_CHECK();
+        } else {
+            points_hessian(h, x, h.hloc.get());
+        }
         if (project_to_psd) psd_project_blocks(h, h.hloc.get());
         auto gath = [&]<int GS>() {
             k_gather_blocks_seg<T, GS><<<xcd_grid(p.n_chunks), GS, 0, h.stream>>>(
