@@ -134,8 +134,8 @@ pfgpu_status pfgpu_set_path(pfgpu_handle *h, int32_t path);
  * mesh at state x (device pointer; 3 timed runs each, after one warm-up) and
  * keeps the fastest.  Candidates: the fused path, the plain path with
  * block-gather workgroups of 128/256/512 threads and Hessian-kernel
- * workgroups of 64/128/256 threads, and the factored path with gather
- * workgroups of 64/128/256/512 threads.  All candidates give identical results
+ * workgroups of 64/128/256 threads, and the factored path with gather sizes
+ * 64/128/256 (its gather chosen by the mesh) and 512 (per contribution).  All candidates give identical results
  * up to the summation order of the path. */
 typedef struct {
     int32_t path, gather_threads, hessian_threads; /* chosen configuration */

@@ -92,7 +92,16 @@ struct GatherPlan {
 // its chunk.
 struct UnitPlan {
     DevBuf chunk_row, udst, bq0, lanes;
-    int n_chunks = 0, threads = 0, split = 1, n_words = 0;
+    int n_chunks = 0, threads = 0, n_words = 0;
+    unsigned grid = 0, grid_grad = 0;
+};
+
+// Wavefront plan of the factored gather (make_wave_plan in plans.hpp): chunk
+// heads, stage positions, block descriptors; state -1 when the mesh has a
+// node with too many incident elements for it.
+struct WavePlan {
+    DevBuf head, dst, desc, long_desc, unused;
+    int n_chunks = 0, n_unused = 0, words = 0, state = 0;
     unsigned grid = 0, grid_grad = 0;
 };
 

@@ -27,7 +27,8 @@ struct pfgpu_handle {
     pfgpu::DevBuf brow_ptr, blk_out;
     std::vector<int32_t> h_contrib_ptr, h_contrib_code;
     pfgpu::GatherPlan blk_plan, fac_plan;
-    pfgpu::UnitPlan unit_plan; // the factored route's row-unit gather
+    pfgpu::WavePlan wave_plan; // the factored route's wavefront gather
+    pfgpu::UnitPlan unit_plan; // its row-unit gather
     // plan of the segmented node-row gather (chunks, padded slots, row metadata)
     pfgpu::DevBuf row_chunk, row_slot, row_meta;
     int n_row_chunks = 0;
@@ -137,6 +138,9 @@ void element_material_vjp(Handle &h, const double *x, const double *p, double *o
 void energy_lame_gradient(Handle &h, const double *x, double *out);
 void plain_shape_vjp(Handle &h, const double *x, const double *p, double *out);
 void ensure_plain_hessian_maps(Handle &h);
+// the wavefront gather of the factored route (gather.hip)
+bool wave_plan_ready(Handle &h);
+void wave_gather(Handle &h, const void *gloc, double *g, void *values);
 void factored_energy_gradient_hessian(Handle &h, const double *x, double *energy, double *g, void *values);
 void factored_node_diagonal(Handle &h, const double *x, void *diag);
 // H v from the factor records in fac_rec (valid only while they belong to x)

@@ -7,6 +7,7 @@
 #include <thread>
 
 #include "dispatch.hpp"
+#include "factors.hpp"
 #include "plans.hpp"
 
 namespace pfgpu {
@@ -39,9 +40,6 @@ template <typename T, int ORDER, int NQ> __device__ __forceinline__ const RefTab
 
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
-
-// Hessian factor record of the factored route (see k_hfactors): values per element
-__host__ __device__ constexpr int fac_size(int nq) { return (11 * nq + 6 + 3) & ~3; }
 
 // the point-independent tail of a factor record, and the record's store
 template <typename T, int NQ> __device__ __forceinline__ void factors_tail(const T *jit, T mu, T w, T (&r)[fac_size(NQ)])
@@ -1634,11 +1632,10 @@ template <typename T, int O, int Q> void launch_factored_gather(Handle &h, Gathe
 
 // the row-unit plan of workgroups of gs threads, split threads per unit
 // (layout at k_gather_units, built by make_unit_plan); false when a node has
-// more incident elements than one chunk holds (the per-contribution gather
-// then serves the handle)
+// more incident elements than one chunk holds
 bool build_unit_plan(Handle &h, UnitPlan &p, int gs, int split)
 {
-    if (p.threads == gs && p.split == split) return true;
+    if (p.threads == gs) return true;
     UnitPlanHost u;
     if (!make_unit_plan(h.pat, h.n_local, h.h_elem_nodes.data(), gs / split, gs, u)) return false;
     // per chunk boundary: first row, first unit, first pattern block
@@ -1662,7 +1659,6 @@ bool build_unit_plan(Handle &h, UnitPlan &p, int gs, int split)
     p.lanes = upload(u.lanes, h.stream);
     p.n_chunks = nc;
     p.threads = gs;
-    p.split = split;
     p.grid = p.grid_grad = 0;
     return true;
 }
@@ -1684,8 +1680,8 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
             if (h.n_cu == 0) PF_HIP(hipDeviceGetAttribute(&h.n_cu, hipDeviceAttributeMultiprocessorCount, h.device));
             int per_cu = 0;
             PF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, GS, size_t(lds)));
-            const int g = std::max(1, h.n_cu) * std::max(1, per_cu);
-            grid = std::min(xcd_grid(p.n_chunks), unsigned((g + N_XCD - 1) / N_XCD * N_XCD));
+            const int n = std::max(1, h.n_cu) * std::max(1, per_cu);
+            grid = std::min(xcd_grid(p.n_chunks), unsigned((n + N_XCD - 1) / N_XCD * N_XCD));
         }
         kern<<<grid, GS, lds, h.stream>>>(p.n_chunks, p.n_words, p.chunk_row.as<int4>(), h.node_ptr.as<int32_t>(),
                                           h.node_inc.as<int32_t>(), h.brow_ptr.as<int32_t>(), p.udst.as<uint16_t>(),
@@ -1693,12 +1689,10 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
                                           static_cast<T *>(values), g);
     };
     auto sized = [&]<bool GRAD>() {
-        if (p.threads == 64)
-            gath.template operator()<64, GRAD, 1>();
-        else if (p.threads == 256)
-            gath.template operator()<256, GRAD, 1>();
-        else
+        if (p.threads == 128)
             gath.template operator()<128, GRAD, 2>();
+        else
+            gath.template operator()<256, GRAD, 1>();
     };
     if (gloc)
         sized.template operator()<true>();
@@ -1707,44 +1701,68 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
     PF_LAUNCH_CHECK();
 }
 
-// the factored route's gather for the tuned workgroup size: the row-unit
-// plan, or the per-contribution plan when a node has too many incident
-// elements for it (or the tuned size is 512)
-bool unit_plan_ready(Handle &h)
+// The factored route's gather.  At gather size 512, the per-contribution
+// gather.  Otherwise the wavefront gather (gather.hip) for meshes of more than
+// wave_units units (node incidences) per CU, and below, or where a node lies in
+// more elements than a wavefront's chunk holds (64 at P2, 128 at P1), the
+// row-unit gather: 64 units in a workgroup of 128 threads, two for each unit
+// (each forms half of its blocks); where a node has more than 64, 256 units in
+// 256 threads, one each; and where that does not fit either (more than 255
+// elements, or P2 FP64, whose staged blocks exceed the 160 KB of LDS), the
+// per-contribution gather.
+//
+// A chunk of the wavefront gather is one wavefront's work from end to end: on
+// small meshes two threads per unit finish sooner, and up to a few chunks per
+// wavefront the last, half-empty round of chunks costs what the gather gains.
+// E + G + H of NeoHookean Kuhn boxes, row units / wavefronts, us: P1 FP64 12.6 /
+// 17.6 at 6^3 cells, 37.7 / 39.3 at 23^3, 66.0 / 62.4 at 32^3, 123 / 109 at
+// 40^3; P1 mixed 20.1 / 21.4 at 20^3, 36.2 / 36.8 at 28^3, 53.2 / 47.1 at 36^3,
+// 195 / 163 at 56^3; P2 FP64 20.5 / 31.5 at 4^3, 70.6 / 72.0 at 16^3, 93.5 /
+// 74.1 at 18^3; P2 mixed 23.1 / 27.3 at 10^3, 42.3 / 43.3 at 16^3, 52.9 / 48.4
+// at 18^3, 450 / 363 at 40^3.  256 units of one thread each took 14.4 us where
+// 64 of two take 12.3 (P1 FP64, 4^3), 24.3 / 19.2 (P2 mixed, 4^3).
+constexpr int wave_units(int order) { return order == 2 ? 1024 : 2048; }
+enum class Gather { wave, units, contributions };
+Gather gather_route(Handle &h)
 {
     if (h.material != MAT_NH && h.material != MAT_LE)
         fail(PFGPU_ERR_UNSUPPORTED, "the factored Hessian covers NeoHookean and linear elasticity");
+    if (h.tune_gather_threads > 256) return Gather::contributions;
+    if (h.n_cu == 0) PF_HIP(hipDeviceGetAttribute(&h.n_cu, hipDeviceAttributeMultiprocessorCount, h.device));
+    if (int64_t(h.n_elements) * h.n_local > int64_t(h.n_cu) * wave_units(h.order) && wave_plan_ready(h))
+        return Gather::wave;
     ensure_plain_hessian_maps(h);
-    // 64: a chunk of 64 units, one thread each; 128: 64 units, two threads
-    // each (in different wavefronts, each forming half of the blocks); 256:
-    // 256 units, one thread each
-    int gs = h.tune_gather_threads;
-    if (gs > 256 || 9 * int64_t(h.pat.n_blocks) >= (int64_t(1) << 31)) return false;
+    if (9 * int64_t(h.pat.n_blocks) >= (int64_t(1) << 31)) return Gather::contributions;
+    if (h.unit_plan.threads || build_unit_plan(h, h.unit_plan, 128, 2)) return Gather::units;
     // dynamic stage + the static tables (row tables, block starts, reference gradients)
-    auto lds = [&](int g) {
-        const int u = g == 128 ? 64 : g;
-        return int64_t(h.value_size()) * u * (h.n_local * 9 + 3) + 8 * (u + 1) + 4 * (u * h.n_local / 2 + 2) + 1024;
-    };
-    // the staged blocks must fit the 160 KB of LDS (FP64 P2 at 256 threads
-    // does not): the largest fitting size at or below the tuned one
-    while (gs > 64 && lds(gs) > 160 * 1024) gs /= 2;
-    if (lds(gs) > 160 * 1024) return false;
-    return build_unit_plan(h, h.unit_plan, gs, gs == 128 ? 2 : 1);
+    const int64_t lds = int64_t(h.value_size()) * 256 * (h.n_local * 9 + 3) + 8 * 257 + 4 * (256 * h.n_local / 2 + 2) + 1024;
+    return lds <= 160 * 1024 && build_unit_plan(h, h.unit_plan, 256, 1) ? Gather::units : Gather::contributions;
+}
+
+// the CSR values (and, with g, the gradient from the local ones in h.loc) from
+// the factor records in h.fac_rec
+template <typename T, int O, int Q> void gather_factored(Handle &h, Gather route, double *g, void *values)
+{
+    if (route == Gather::wave) {
+        wave_gather(h, g ? h.loc.get() : nullptr, g, values);
+    } else if (route == Gather::units) {
+        launch_unit_gather<T, O, Q>(h, h.unit_plan, g ? h.loc.as<T>() : nullptr, g, values);
+    } else {
+        if (g) gather_rows(h, h.loc.get(), g);
+        launch_factored_gather<T, O, Q>(h, factored_plan(h), values);
+    }
 }
 
 void factored_hessian(Handle &h, const double *x, void *values)
 {
-    const bool units = unit_plan_ready(h);
-    GatherPlan *p = units ? nullptr : &factored_plan(h);
+    const Gather route = gather_route(h);
+    if (route == Gather::contributions) factored_plan(h);
     dispatch<true>(h, [&]<typename T, int O, int Q, int M>() {
         if constexpr (M == MAT_NH || M == MAT_LE) {
             h.fac_rec.reserve(sizeof(T) * size_t(h.n_elements) * fac_size(Q));
             k_hfactors<T, O, Q, M><<<grid_for(h.n_elements, 64), 64, 0, h.stream>>>(h.mesh<T>(), x, h.fac_rec.as<T>());
             PF_LAUNCH_CHECK();
-            if (units)
-                launch_unit_gather<T, O, Q>(h, h.unit_plan, nullptr, nullptr, values);
-            else
-                launch_factored_gather<T, O, Q>(h, *p, values);
+            gather_factored<T, O, Q>(h, route, nullptr, values);
         }
     });
 }
@@ -1753,8 +1771,8 @@ void factored_hessian(Handle &h, const double *x, void *values)
 // gradient, the energy partials and the Hessian factor records
 void factored_energy_gradient_hessian(Handle &h, const double *x, double *energy, double *g, void *values)
 {
-    const bool units = unit_plan_ready(h);
-    GatherPlan *p = units ? nullptr : &factored_plan(h);
+    const Gather route = gather_route(h);
+    if (route == Gather::contributions) factored_plan(h);
     const unsigned grid = grid_for(h.n_elements, 64);
     h.loc.reserve(h.value_size() * size_t(h.n_elements) * h.n_local * 3);
     if (energy) h.partial.reserve(sizeof(double) * grid);
@@ -1764,13 +1782,8 @@ void factored_energy_gradient_hessian(Handle &h, const double *x, double *energy
             k_grad_factors<T, O, Q, M><<<grid, 64, 0, h.stream>>>(
                 h.mesh<T>(), x, h.loc.as<T>(), energy ? h.partial.as<double>() : nullptr, h.fac_rec.as<T>());
             PF_LAUNCH_CHECK();
-            if (units) {
-                // the gradient rows are summed by the same pass
-                launch_unit_gather<T, O, Q>(h, h.unit_plan, h.loc.as<T>(), g, values);
-            } else {
-                gather_rows(h, h.loc.get(), g);
-                launch_factored_gather<T, O, Q>(h, *p, values);
-            }
+            // the gradient rows are summed by the same pass
+            gather_factored<T, O, Q>(h, route, g, values);
             if (energy) sum_doubles(h, h.partial.as<double>(), int(grid), energy);
         }
     });

@@ -3,6 +3,7 @@
 // only, so that tests can build and check the plans on the CPU.
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <thread>
 
 #include "plans.hpp"
@@ -153,6 +154,222 @@ bool make_unit_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
     out.udst = std::move(dst);
     out.bq0 = std::move(q0);
     out.lanes = std::move(lanes);
+    return true;
+}
+
+namespace {
+
+// the stage that a chunk's contribution counts (descending) need
+struct WaveShape {
+    int n_long = 0, n_groups = 0, long_base = 0, max_pieces = 0, words = 0;
+    uint8_t count[WAVE_GROUPS] = {};
+    int base[WAVE_GROUPS] = {};
+};
+WaveShape wave_shape(const std::vector<int32_t> &cnt)
+{
+    WaveShape s;
+    const int nb = int(cnt.size()), out_words = (4 * nb + 7) / 8 * 8;
+    int pieces = 0;
+    for (; s.n_long < nb && cnt[size_t(s.n_long)] > WAVE_SHORT; ++s.n_long) {
+        const int p = (cnt[size_t(s.n_long)] + WAVE_SHORT - 1) / WAVE_SHORT;
+        pieces += p;
+        s.max_pieces = std::max(s.max_pieces, p);
+    }
+    int word = 0;
+    for (int k = s.n_long; k < nb; k += 64, ++s.n_groups) {
+        const int most = cnt[size_t(k)], least = cnt[size_t(std::min(k + 63, nb - 1))];
+        s.base[s.n_groups] = word;
+        s.count[s.n_groups] = uint8_t(most | least << 4);
+        word += 192 * most + 8;
+        if (s.n_groups == 0) word = std::max(word, out_words);
+    }
+    s.long_base = std::max(word, out_words);
+    s.words = s.long_base + (pieces + 7) / 8 * 192;
+    return s;
+}
+
+} // namespace
+
+bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
+                    int value_size, WavePlanHost &out)
+{
+    const std::vector<int32_t> &np = pat.node_ptr, &ni = pat.node_inc, &bp = pat.brow_ptr, &bc = pat.bcol;
+    const int NB = n_local, N = pat.n_nodes, cap = 64 * rounds;
+    // contributions per block, and every unit's block positions in its row
+    std::vector<uint8_t> count(size_t(pat.n_blocks));
+    std::vector<uint16_t> upos(size_t(np[size_t(N)]) * NB);
+    std::atomic<bool> fits{true};
+    const int nt = int(std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+    auto parallel = [&](int n, auto &&f) {
+        std::vector<std::thread> pool;
+        for (int t = 0; t < nt; ++t) pool.emplace_back(f, int(int64_t(n) * t / nt), int(int64_t(n) * (t + 1) / nt));
+        for (std::thread &th : pool) th.join();
+    };
+    parallel(N, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            const int32_t r0 = bp[size_t(i)], deg = bp[size_t(i) + 1] - r0;
+            if (np[size_t(i) + 1] - np[size_t(i)] > cap || deg > WAVE_BLOCKS) {
+                fits = false;
+                return;
+            }
+            const int32_t *cols = bc.data() + r0;
+            for (int32_t u = np[size_t(i)]; u < np[size_t(i) + 1]; ++u) {
+                const int32_t e = ni[size_t(u)] / NB;
+                for (int b = 0; b < NB; ++b) {
+                    const int p = int(std::lower_bound(cols, cols + deg, elem_nodes[size_t(e) * NB + b]) - cols);
+                    upos[size_t(u) * NB + b] = uint16_t(p);
+                    count[size_t(r0 + p)]++;
+                }
+            }
+        }
+    });
+    if (!fits) return false;
+    // chunks of whole rows: as many nodes as the cheap limits allow, given
+    // back while the chunk's stage exceeds the cap
+    std::vector<WaveHead> head;
+    std::vector<int32_t> cnt;
+    int64_t nw = 0, nl = 0;
+    for (int i = 0; i < N;) {
+        int j = i + 1;
+        while (j < N && j - i < WAVE_ROWS && np[size_t(j) + 1] - np[size_t(i)] <= cap &&
+               bp[size_t(j) + 1] - bp[size_t(i)] <= WAVE_BLOCKS)
+            ++j;
+        WaveShape s;
+        while (true) {
+            cnt.assign(count.begin() + bp[size_t(i)], count.begin() + bp[size_t(j)]);
+            std::sort(cnt.begin(), cnt.end(), std::greater<int32_t>());
+            s = wave_shape(cnt);
+            if (j == i + 1 || (s.words <= word_cap && s.n_long <= 64)) break;
+            --j;
+        }
+        if (s.n_long > 64) return false;
+        WaveHead h{};
+        h.row0 = i;
+        h.unit0 = np[size_t(i)];
+        h.blk0 = bp[size_t(i)];
+        h.desc0 = int32_t(nw);
+        h.n_rows = j - i;
+        h.n_units = np[size_t(j)] - h.unit0;
+        h.n_blocks = bp[size_t(j)] - h.blk0;
+        h.n_long = s.n_long;
+        h.long0 = int32_t(nl);
+        h.long_base = s.long_base;
+        h.n_groups = s.n_groups;
+        h.max_pieces = s.max_pieces;
+        std::copy(s.count, s.count + WAVE_GROUPS, h.count);
+        if (h.n_blocks) {
+            nw += 64 * s.n_groups;
+            nl += s.n_long;
+            if (nw >= (int64_t(1) << 31) || s.words * value_size > 65536) return false;
+            out.max_words = std::max(out.max_words, s.words);
+            head.push_back(h);
+        } else {
+            for (int k = i; k < j; ++k) out.unused.push_back(k);
+        }
+        i = j;
+    }
+    const int nc = int(head.size());
+    std::vector<uint32_t> desc(static_cast<size_t>(nw), 0), long_desc(size_t(2 * nl));
+    std::vector<uint16_t> dst(size_t(nc) * size_t(cap) * size_t(NB), 0);
+    parallel(nc, [&](int c0, int c1) {
+        // per output block: its contributions (unit, b), in unit order
+        std::vector<int32_t> ptr, list, order, next, sorted, row_of, pos(size_t(cap) * size_t(NB));
+        for (int ci = c0; ci < c1; ++ci) {
+            WaveHead &h = head[size_t(ci)];
+            const int nb = h.n_blocks, B0 = h.blk0;
+            ptr.assign(size_t(nb) + 1, 0);
+            for (int k = 0; k < nb; ++k) ptr[size_t(k) + 1] = ptr[size_t(k)] + count[size_t(B0 + k)];
+            list.resize(size_t(ptr[size_t(nb)]));
+            order.resize(size_t(nb));
+            row_of.resize(size_t(nb));
+            next.assign(ptr.begin(), ptr.end() - 1);
+            for (int i = h.row0; i < h.row0 + h.n_rows; ++i) {
+                for (int32_t b = bp[size_t(i)]; b < bp[size_t(i) + 1]; ++b) row_of[size_t(b - B0)] = i - h.row0;
+                for (int32_t u = np[size_t(i)]; u < np[size_t(i) + 1]; ++u)
+                    for (int b = 0; b < NB; ++b) {
+                        const int k = bp[size_t(i)] - B0 + upos[size_t(u) * NB + b];
+                        list[size_t(next[size_t(k)]++)] = (u - h.unit0) * NB + b;
+                    }
+            }
+            for (int k = 0; k < nb; ++k) order[size_t(k)] = k;
+            std::stable_sort(order.begin(), order.end(),
+                             [&](int32_t x, int32_t y) { return count[size_t(B0 + x)] > count[size_t(B0 + y)]; });
+            sorted.resize(size_t(nb));
+            for (int j = 0; j < nb; ++j) sorted[size_t(j)] = count[size_t(B0 + order[size_t(j)])];
+            const WaveShape s = wave_shape(sorted);
+            auto word = [&](int k) { return uint32_t(k) << 4 | uint32_t(4 * row_of[size_t(k)]) << 14; };
+            int pieces = 0;
+            for (int j = 0; j < h.n_long; ++j) {
+                const int k = order[size_t(j)], n = sorted[size_t(j)];
+                long_desc[2 * size_t(h.long0 + j)] = word(k);
+                long_desc[2 * size_t(h.long0 + j) + 1] = uint32_t(pieces) | uint32_t(n) << 16;
+                for (int q = 0; q < n; ++q) {
+                    const int p = pieces + q / WAVE_SHORT;
+                    pos[size_t(list[size_t(ptr[size_t(k)] + q)])] = h.long_base + p / 8 * 192 + p % 8 * WAVE_SHORT + q % WAVE_SHORT;
+                }
+                pieces += (n + WAVE_SHORT - 1) / WAVE_SHORT;
+            }
+            // banks[level][instruction and half wavefront]: the banks used
+            // more than `level` times; octet[group][lanes / 8]: the output
+            // banks (blocks modulo 8) its eight lanes store to
+            uint32_t banks[3][40] = {};
+            uint8_t octet[WAVE_GROUPS][8] = {};
+            auto instr = [&](int v) { return (v % NB * rounds + v / NB / 64) * 2 + v / NB % 64 / 32; };
+            uint64_t free_lanes[WAVE_GROUPS];
+            int least[WAVE_GROUPS];
+            std::fill(free_lanes, free_lanes + WAVE_GROUPS, ~uint64_t(0));
+            std::fill(least, least + WAVE_GROUPS, WAVE_SHORT);
+            uint32_t *dc = desc.data() + h.desc0;
+            for (int j = h.n_long; j < nb; ++j) {
+                const int k = order[size_t(j)], n = sorted[size_t(j)];
+                int best = 8, to = -1, lane = 0;
+                for (int g = 0; g < h.n_groups && best > 0; ++g) {
+                    if (n > (s.count[g] & 15) || (n < s.count[g] >> 4 && to >= 0)) continue;
+                    // banks taken (once, twice, three times) by the instructions
+                    // of the block's contributions, shifted back to its lane
+                    uint32_t used[4] = {0, 0, 0, 0};
+                    for (int q = 0; q < n; ++q) {
+                        const int x = instr(list[size_t(ptr[size_t(k)] + q)]), by = (s.base[g] + q) % 32;
+                        for (int lv = 0; lv < 3; ++lv) used[lv] |= by ? banks[lv][x] >> by | banks[lv][x] << (32 - by) : banks[lv][x];
+                    }
+                    uint64_t clash = 0;
+                    for (int o = 0; o < 8; ++o)
+                        if (octet[g][o] >> (k % 8) & 1) clash |= uint64_t(255) << (8 * o);
+                    for (int cost = 0; cost < best; ++cost) {
+                        const uint32_t u = used[cost / 2];
+                        uint64_t pick = free_lanes[g] & ~(uint64_t(u) << 32 | u);
+                        if (cost % 2 == 0) pick &= ~clash;
+                        if (pick) {
+                            best = cost;
+                            to = g;
+                            lane = __builtin_ctzll(pick);
+                        }
+                    }
+                }
+                free_lanes[to] &= ~(uint64_t(1) << lane);
+                octet[to][lane / 8] |= uint8_t(1 << (k % 8));
+                least[to] = std::min(least[to], n);
+                for (int q = 0; q < n; ++q) {
+                    const int v = list[size_t(ptr[size_t(k)] + q)], x = instr(v), w = s.base[to] + WAVE_STEP * q + lane;
+                    const uint32_t bit = uint32_t(1) << (w % 32);
+                    for (int lv = 2; lv > 0; --lv) banks[lv][x] |= banks[lv - 1][x] & bit;
+                    banks[0][x] |= bit;
+                    pos[size_t(v)] = w;
+                }
+                dc[64 * to + lane] = word(k) | uint32_t(n);
+            }
+            for (int g = 0; g < h.n_groups; ++g) h.count[g] = uint8_t((h.count[g] & 15) | least[g] << 4);
+            uint16_t *d = dst.data() + size_t(ci) * size_t(cap) * size_t(NB);
+            for (int v = 0; v < h.n_units; ++v)
+                for (int b = 0; b < NB; ++b)
+                    // pairs of positions share a word, words of the lanes adjacent
+                    d[((size_t(v / 64) * (NB / 2) + b / 2) * 64 + v % 64) * 2 + b % 2] = uint16_t(pos[size_t(v) * NB + b] * value_size);
+        }
+    });
+    out.head = std::move(head);
+    out.dst = std::move(dst);
+    out.desc = std::move(desc);
+    out.long_desc = std::move(long_desc);
     return true;
 }
 

@@ -42,6 +42,55 @@ struct UnitPlanHost {
 bool make_unit_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int gs, int n_lanes,
                     UnitPlanHost &out);
 
+// Wavefront plan of the factored gather (k_gather_wave in gather.hip): a
+// chunk is a run of whole node rows with at most 64 rounds units, WAVE_ROWS
+// rows and WAVE_BLOCKS pattern blocks, gathered by one wavefront.  A unit is a
+// node incidence as above; unit v of the chunk is formed by lane v % 64 of
+// round v / 64.
+//
+// The wavefront stages the three entries of a row of every contribution in
+// LDS and adds them by descending count of contributions, so that its lanes
+// add alike.  The short blocks (at most WAVE_SHORT contributions) are dealt
+// 64 at a time to the lanes; entry n of contribution k of the block on lane l
+// of group g sits at word base_g + WAVE_STEP k + 64 n + l: the lanes read
+// their sums without bank conflicts and with no index arithmetic, and a group
+// whose largest count is c takes 192 c + 8 words.  The lane of a block, and
+// its group where several hold its count, are chosen so that the words one
+// store instruction fills lie in different LDS banks as far as possible;
+// WAVE_STEP = 193 instead of 192 parts the contributions that one block gets
+// from one instruction (P2: 1.9 cycles per store of 32 lanes where the first
+// free lane takes 3.4 and the choice without the extra word 2.8; P1: 2.0
+// where it takes 3.8).  The long blocks' contributions follow from word
+// long_base in pieces of WAVE_SHORT, eight pieces per 192 words.  The sums go
+// to an output area of 4 words per block that overlaps group 0; group 1
+// starts behind it.
+//
+// dst holds, per chunk, round and lane, the stage positions (entry 0, in
+// bytes) of the contributions b = 0 .. n_local - 1 of the lane's unit, 0 past
+// the last unit.  desc holds per chunk one word per lane of its groups,
+// count | block << 4 | 4 row << 14 (block and row chunk-local; count 0 for a
+// lane without a block), and long_desc two words per long block: block << 4 |
+// 4 row << 14, and its first piece | contributions << 16.
+constexpr int WAVE_SHORT = 8, WAVE_ROWS = 63, WAVE_BLOCKS = 1023, WAVE_GROUPS = 16, WAVE_STEP = 193;
+struct WaveHead {
+    int32_t row0, unit0, blk0, desc0; // first row, unit, pattern block and descriptor of the chunk
+    int32_t n_rows, n_units, n_blocks, n_long;
+    int32_t long0, long_base, n_groups, max_pieces; // first long block; most pieces of one
+    uint8_t count[WAVE_GROUPS];                     // per group: largest count | smallest count << 4
+};
+struct WavePlanHost {
+    std::vector<WaveHead> head; // every chunk holds at least one block
+    std::vector<uint16_t> dst;
+    std::vector<uint32_t> desc, long_desc;
+    std::vector<int32_t> unused; // nodes outside the chunks: no element uses them
+    int max_words = 0;           // stage words of the largest chunk
+};
+// word_cap: stage words of a chunk of more than one node; value_size: bytes of
+// an entry.  False when a row has more than 64 rounds (at most 2) units,
+// WAVE_BLOCKS blocks or 64 long blocks.
+bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
+                    int value_size, WavePlanHost &out);
+
 // Chunks of consecutive outputs 0 .. n-1, output i gathering the
 // contributions ptr[i] .. ptr[i+1]-1: a chunk holds at most cap
 // contributions; c = chunk starts plus n.  False when one output alone has
