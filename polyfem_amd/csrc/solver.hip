@@ -44,22 +44,35 @@ constexpr int SPMV_LANES = PF_SPMV_LANES; // lanes per block row of the block-sp
 // scalar slots of the CG workspace (r.z: preconditioned residual product)
 // S_FLAG: 0 while the CG runs, 1 stopped on non-positive curvature, 2 stopped
 // at the tolerance (r.r <= S_TOL); S_ITER counts the updates taken
-enum { S_RR, S_PQ, S_ALPHA, S_BETA, S_RZ, S_FLAG, S_B2, S_GD, S_E0, S_E1, S_M, S_F, S_TOL, S_ITER, S_COUNT };
+// S_OLD, S_STOP: r.z and the flag of the running iteration as the update kernel
+// leaves them for the direction kernel, which writes S_RZ and S_FLAG
+enum { S_RR, S_PQ, S_ALPHA, S_BETA, S_RZ, S_FLAG, S_B2, S_GD, S_E0, S_E1, S_M, S_F, S_TOL, S_ITER, S_OLD, S_STOP, S_COUNT };
 enum { CG_RUNNING = 0, CG_CURVATURE = 1, CG_TOLERANCE = 2 };
 
+// the sum over the workgroup, in every thread: the tree s[t] += s[t + w],
+// w = BLOCK / 2 .. 1, its last six levels inside the first wavefront (one
+// barrier before the result where a level each takes eight)
 __device__ double block_reduce(double v, double *sh)
 {
+    static_assert(BLOCK == 256, "two levels of the tree lie above a wavefront's");
     const int t = threadIdx.x;
-    sh[t] = v;
+    if (t < BLOCK) sh[t] = v;
     __syncthreads();
-    for (int w = BLOCK / 2; w > 0; w >>= 1) {
-        if (t < w) sh[t] += sh[t + w];
-        __syncthreads();
+    if (t < 64) {
+        double r = (sh[t] + sh[t + 128]) + (sh[t + 64] + sh[t + 192]);
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) r += __shfl_down(r, w, 64);
+        if (t == 0) sh[0] = r;
     }
+    __syncthreads();
     const double r = sh[0];
     __syncthreads();
     return r;
 }
+
+// blocks that hold items 0 .. n-1 under the fixed stride of DOT_BLOCKS BLOCK
+// (the partials of the others would be zero)
+inline unsigned dot_blocks(int n) { return std::min(unsigned(DOT_BLOCKS), grid_for(n)); }
 
 // per-block partial of sum_i a_i b_i over free dofs (mask: 1 = fixed)
 __global__ __launch_bounds__(BLOCK) void k_dot_partials(const double *__restrict__ a, const double *__restrict__ b,
@@ -69,39 +82,24 @@ __global__ __launch_bounds__(BLOCK) void k_dot_partials(const double *__restrict
     double v = 0;
     for (int i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += DOT_BLOCKS * BLOCK)
         if (!fixed || !fixed[i]) v = fma(a[i], b[i], v);
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = BLOCK / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+    v = block_reduce(v, s);
+    if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
-// one block: fixed-order sum of the DOT_BLOCKS partials into scal[slot], then
-// the scalar bookkeeping of the step that follows
-enum { AFTER_NONE, AFTER_ALPHA };
-__device__ double sum_partials(const double *__restrict__ part, double *sh)
+// fixed-order sum of the first n of the DOT_BLOCKS partials
+__device__ double sum_partials(const double *__restrict__ part, int n, double *sh)
 {
     double a = 0;
-    for (int k = threadIdx.x; k < DOT_BLOCKS; k += BLOCK) a += part[k];
+    for (int k = threadIdx.x; k < n; k += BLOCK) a += part[k];
     return block_reduce(a, sh);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_finish_dot(const double *__restrict__ part, double *__restrict__ scal, int slot,
-                                                      int after)
+// one block: the sum of the partials into scal[slot]
+__global__ __launch_bounds__(BLOCK) void k_finish_dot(const double *__restrict__ part, int n, double *__restrict__ scal, int slot)
 {
     __shared__ double s[BLOCK];
-    const double v = sum_partials(part, s);
-    if (threadIdx.x != 0) return;
-    scal[slot] = v;
-    if (after == AFTER_ALPHA) {
-        // alpha = r.z / p.Hp; a non-positive curvature stops the iteration
-        const double rz = scal[S_RZ];
-        const bool ok = v > 0.0 && rz > 0.0 && scal[S_FLAG] == 0.0;
-        if (!(v > 0.0) && rz > 0.0 && scal[S_FLAG] == 0.0) scal[S_FLAG] = CG_CURVATURE;
-        scal[S_ALPHA] = ok ? rz / v : 0.0;
-    }
+    const double v = sum_partials(part, n, s);
+    if (threadIdx.x == 0) scal[slot] = v;
 }
 
 // z = P r for one node: P the inverse of the node's 3x3 diagonal block (symmetric,
@@ -120,11 +118,11 @@ __device__ inline void precondition(const float *__restrict__ pinv, int64_t i, c
     z[2] = fma(c, r[0], fma(e, r[1], f * r[2]));
 }
 
-// PCG start: y = 0, r = b on free dofs, z = P r, p = z; partials of r.z and r.r
+// PCG start: y = 0, r = b on free dofs, p = z = P r; partials of r.z and r.r
 __global__ __launch_bounds__(BLOCK) void k_pcg_start(int n_nodes, const double *__restrict__ b,
                                                      const uint8_t *__restrict__ fixed, const float *__restrict__ pinv,
                                                      double *__restrict__ y, double *__restrict__ r,
-                                                     double *__restrict__ z, double *__restrict__ p,
+                                                     double *__restrict__ p,
                                                      double *__restrict__ part_rz, double *__restrict__ part_rr)
 {
     __shared__ double sh[BLOCK];
@@ -139,7 +137,6 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_start(int n_nodes, const double *
         for (int d = 0; d < 3; ++d) {
             y[o + d] = 0.0;
             r[o + d] = ri[d];
-            z[o + d] = zi[d];
             p[o + d] = zi[d];
             rz = fma(ri[d], zi[d], rz);
             rr = fma(ri[d], ri[d], rr);
@@ -152,40 +149,49 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_start(int n_nodes, const double *
     }
 }
 
-// y += alpha p, r -= alpha q on free dofs; z = P r; partials of r.z and r.r
-__global__ __launch_bounds__(BLOCK) void k_pcg_update(int n_nodes, double *__restrict__ y, double *__restrict__ r,
-                                                      double *__restrict__ z, const double *__restrict__ p,
+// alpha = r.z / p.Hp from the p.Hp partials of n_pq blocks (a non-positive
+// curvature stops the iteration), then r -= alpha q on free dofs; partials of
+// r.z, z = P r, and r.r.  Every block sums the partials again, in the same
+// order: at most 8 KB from L2 instead of a launch of one block between the two
+// kernels.  An iteration at these sizes is launches and latency: seven kernels
+// of 42 us became five of 34 on 284,000 dofs (P2, matrix-free), six of 20 us
+// four of 13 on 10,000 (P1, assembled).
+__global__ __launch_bounds__(BLOCK) void k_pcg_update(int n_nodes, int n_pq, double *__restrict__ r,
                                                       const double *__restrict__ q, const uint8_t *__restrict__ fixed,
-                                                      const float *__restrict__ pinv, const double *__restrict__ scal,
-                                                      double *__restrict__ part_rz, double *__restrict__ part_rr)
+                                                      const float *__restrict__ pinv, double *__restrict__ scal,
+                                                      const double *__restrict__ part_pq, double *__restrict__ part_rz,
+                                                      double *__restrict__ part_rr)
 {
     __shared__ double sh[BLOCK];
-    const double a = scal[S_ALPHA];
+    const double v = sum_partials(part_pq, n_pq, sh), old = scal[S_RZ], flag = scal[S_FLAG];
+    const double a = v > 0.0 && old > 0.0 && flag == 0.0 ? old / v : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        scal[S_PQ] = v;
+        scal[S_ALPHA] = a;
+        scal[S_OLD] = old;
+        scal[S_STOP] = !(v > 0.0) && old > 0.0 && flag == 0.0 ? double(CG_CURVATURE) : flag;
+    }
     double rz = 0, rr = 0;
     for (int i = blockIdx.x * BLOCK + threadIdx.x; i < n_nodes; i += DOT_BLOCKS * BLOCK) {
         const int64_t o = 3 * int64_t(i);
         // every load of the node first, then the masked update
-        double ri[3], zi[3], pi[3], qi[3], yi[3];
+        double ri[3], zi[3], qi[3];
         bool upd[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             ri[d] = r[o + d];
-            pi[d] = p[o + d];
             qi[d] = q[o + d];
-            yi[d] = y[o + d];
             upd[d] = a != 0.0 && !(fixed && fixed[o + d]);
         }
 #pragma unroll
         for (int d = 0; d < 3; ++d)
             if (upd[d]) {
-                y[o + d] = fma(a, pi[d], yi[d]);
                 ri[d] = fma(-a, qi[d], ri[d]);
                 r[o + d] = ri[d];
             }
         precondition(pinv, i, ri, zi);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            z[o + d] = zi[d];
             rz = fma(ri[d], zi[d], rz);
             rr = fma(ri[d], ri[d], rr);
         }
@@ -197,30 +203,62 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_update(int n_nodes, double *__res
     }
 }
 
-// sums of the r.z and r.r partials; at the start they set r.z and r.r, after an
-// update they also give beta = r'.z' / r.z (zero once the iteration has stopped)
-__global__ __launch_bounds__(BLOCK) void k_finish_pcg(const double *__restrict__ part_rz, const double *__restrict__ part_rr,
-                                                      double *__restrict__ scal, int start)
+// the start's r.z and r.r from their partials
+__global__ __launch_bounds__(BLOCK) void k_start_pcg(const double *__restrict__ part_rz, const double *__restrict__ part_rr,
+                                                     int n, double *__restrict__ scal)
 {
     __shared__ double s[BLOCK];
-    const double rz = sum_partials(part_rz, s), rr = sum_partials(part_rr, s);
+    const double rz = sum_partials(part_rz, n, s), rr = sum_partials(part_rr, n, s);
     if (threadIdx.x != 0) return;
-    if (start) {
-        scal[S_RZ] = rz;
-        scal[S_RR] = rr;
-        scal[S_FLAG] = CG_RUNNING;
-        scal[S_ITER] = 0.0;
-        return;
+    scal[S_RZ] = rz;
+    scal[S_RR] = rr;
+    scal[S_FLAG] = CG_RUNNING;
+    scal[S_ITER] = 0.0;
+}
+
+// beta = r'.z' / r.z from the update's partials (zero once the iteration has
+// stopped), then y += alpha p on free dofs and p = z + beta p, z = P r formed
+// again from r (an FP32 triangle instead of a written and read vector).  Every
+// block sums the partials (k_pcg_update); the first one keeps the state.
+__global__ __launch_bounds__(BLOCK) void k_cg_direction(int n_nodes, double *__restrict__ y, double *__restrict__ p,
+                                                        const double *__restrict__ r, const uint8_t *__restrict__ fixed,
+                                                        const float *__restrict__ pinv, double *__restrict__ scal,
+                                                        const double *__restrict__ part_rz, const double *__restrict__ part_rr)
+{
+    __shared__ double s[BLOCK];
+    const double old = scal[S_OLD], stop = scal[S_STOP], a = scal[S_ALPHA];
+    const bool live = stop == 0.0 && old > 0.0;
+    const double rz = sum_partials(part_rz, int(gridDim.x), s), beta = live ? rz / old : 0.0;
+    if (blockIdx.x == 0) { // uniform over the workgroup
+        const double rr = sum_partials(part_rr, int(gridDim.x), s);
+        if (threadIdx.x == 0) {
+            scal[S_BETA] = beta;
+            if (stop == 0.0) {
+                scal[S_RZ] = rz;
+                scal[S_RR] = rr;
+                if (live) scal[S_ITER] += 1.0;
+            }
+            // the iteration stops where it meets the tolerance
+            scal[S_FLAG] = stop == 0.0 && rr <= scal[S_TOL] ? double(CG_TOLERANCE) : stop;
+        }
     }
-    const double old = scal[S_RZ];
-    const bool live = scal[S_FLAG] == 0.0 && old > 0.0;
-    scal[S_BETA] = live ? rz / old : 0.0;
-    if (scal[S_FLAG] == 0.0) {
-        scal[S_RZ] = rz;
-        scal[S_RR] = rr;
-        if (live) scal[S_ITER] += 1.0;
-        // the iteration stops where it meets the tolerance
-        if (rr <= scal[S_TOL]) scal[S_FLAG] = CG_TOLERANCE;
+    for (int i = blockIdx.x * BLOCK + threadIdx.x; i < n_nodes; i += DOT_BLOCKS * BLOCK) {
+        const int64_t o = 3 * int64_t(i);
+        double ri[3], zi[3], pi[3], yi[3];
+        bool upd[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            ri[d] = r[o + d];
+            pi[d] = p[o + d];
+            yi[d] = y[o + d];
+            upd[d] = a != 0.0 && !(fixed && fixed[o + d]);
+        }
+        precondition(pinv, i, ri, zi);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (upd[d]) y[o + d] = fma(a, pi[d], yi[d]);
+            p[o + d] = fma(beta, pi[d], zi[d]);
+        }
     }
 }
 
@@ -345,15 +383,6 @@ __global__ __launch_bounds__(BLOCK) void k_mask(double *__restrict__ q, const ui
     if (i < n && fixed && fixed[i]) q[i] = 0.0;
 }
 
-// p = z + beta p
-__global__ __launch_bounds__(BLOCK) void k_cg_direction(double *__restrict__ p, const double *__restrict__ z,
-                                                        const double *__restrict__ scal, int n)
-{
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    p[i] = fma(scal[S_BETA], p[i], z[i]);
-}
-
 __global__ void k_set_scalar(double *__restrict__ scal, int slot, double v) { scal[slot] = v; }
 
 // out = x + a d (a read from the host argument), or -v on free dofs
@@ -471,22 +500,23 @@ __global__ __launch_bounds__(BLOCK) void k_axpy(double *__restrict__ out, double
 }
 
 struct Work {
-    double *r, *p, *q, *y, *g, *xt, *d, *t, *mt, *z, *scal, *part, *part2;
+    double *r, *p, *q, *y, *g, *xt, *d, *t, *mt, *scal, *part, *part2, *part3;
 };
 
 Work workspace(Handle &h)
 {
     const size_t n = size_t(h.n_dofs);
-    h.sv.reserve(sizeof(double) * (10 * n + S_COUNT + 2 * DOT_BLOCKS));
-    double *b = h.sv.as<double>();
-    return Work{b,         b + n,     b + 2 * n,           b + 3 * n, b + 4 * n, b + 5 * n, b + 6 * n, b + 7 * n, b + 8 * n,
-                b + 9 * n, b + 10 * n, b + 10 * n + S_COUNT, b + 10 * n + S_COUNT + DOT_BLOCKS};
+    h.sv.reserve(sizeof(double) * (9 * n + S_COUNT + 3 * DOT_BLOCKS));
+    double *b = h.sv.as<double>(), *scal = b + 9 * n, *part = scal + S_COUNT;
+    return Work{b,         b + n,     b + 2 * n, b + 3 * n, b + 4 * n,         b + 5 * n,           b + 6 * n,
+                b + 7 * n, b + 8 * n, scal,      part,      part + DOT_BLOCKS, part + 2 * DOT_BLOCKS};
 }
 
-void dot(Handle &h, const Work &w, const double *a, const double *b, const uint8_t *fixed, int slot, int after)
+void dot(Handle &h, const Work &w, const double *a, const double *b, const uint8_t *fixed, int slot)
 {
-    k_dot_partials<<<DOT_BLOCKS, BLOCK, 0, h.stream>>>(a, b, fixed, h.n_dofs, w.part);
-    k_finish_dot<<<1, BLOCK, 0, h.stream>>>(w.part, w.scal, slot, after);
+    const unsigned n = dot_blocks(h.n_dofs);
+    k_dot_partials<<<n, BLOCK, 0, h.stream>>>(a, b, fixed, h.n_dofs, w.part);
+    k_finish_dot<<<1, BLOCK, 0, h.stream>>>(w.part, int(n), w.scal, slot);
 }
 
 double read_scalar(Handle &h, const Work &w, int slot)
@@ -660,9 +690,9 @@ const float *precond(const Handle &h) { return h.op_valid && h.op_precond ? h.pi
 // PCG start from b (a fixed kernel sequence)
 void cg_start(Handle &h, const Work &w, const uint8_t *fixed, const double *b)
 {
-    k_pcg_start<<<DOT_BLOCKS, BLOCK, 0, h.stream>>>(h.n_nodes, b, fixed, precond(h), w.y, w.r, w.z, w.p, w.part,
-                                                    w.part2);
-    k_finish_pcg<<<1, BLOCK, 0, h.stream>>>(w.part, w.part2, w.scal, 1);
+    const unsigned n = dot_blocks(h.n_nodes);
+    k_pcg_start<<<n, BLOCK, 0, h.stream>>>(h.n_nodes, b, fixed, precond(h), w.y, w.r, w.p, w.part, w.part2);
+    k_start_pcg<<<1, BLOCK, 0, h.stream>>>(w.part, w.part2, int(n), w.scal);
     PF_LAUNCH_CHECK();
 }
 
@@ -670,11 +700,10 @@ void cg_start(Handle &h, const Work &w, const uint8_t *fixed, const double *b)
 void cg_iteration(Handle &h, const Work &w, const double *x, const uint8_t *fixed)
 {
     hvp_any(h, x, w.p, w.q);
-    dot(h, w, w.p, w.q, fixed, S_PQ, AFTER_ALPHA);
-    k_pcg_update<<<DOT_BLOCKS, BLOCK, 0, h.stream>>>(h.n_nodes, w.y, w.r, w.z, w.p, w.q, fixed, precond(h), w.scal,
-                                                     w.part, w.part2);
-    k_finish_pcg<<<1, BLOCK, 0, h.stream>>>(w.part, w.part2, w.scal, 0);
-    k_cg_direction<<<grid_for(h.n_dofs), BLOCK, 0, h.stream>>>(w.p, w.z, w.scal, h.n_dofs);
+    const unsigned n = dot_blocks(h.n_dofs), nn = dot_blocks(h.n_nodes);
+    k_dot_partials<<<n, BLOCK, 0, h.stream>>>(w.p, w.q, fixed, h.n_dofs, w.part);
+    k_pcg_update<<<nn, BLOCK, 0, h.stream>>>(h.n_nodes, int(n), w.r, w.q, fixed, precond(h), w.scal, w.part, w.part2, w.part3);
+    k_cg_direction<<<nn, BLOCK, 0, h.stream>>>(h.n_nodes, w.y, w.p, w.r, fixed, precond(h), w.scal, w.part2, w.part3);
     PF_LAUNCH_CHECK();
 }
 
@@ -688,9 +717,9 @@ void objective_energy(Handle &h, const Work &w, const double *x, int slot)
         k_mass_apply<<<grid_for(h.n_nodes, BLOCK / SPMV_LANES), BLOCK, 0, h.stream>>>(h.n_nodes, h.brow_ptr.as<int32_t>(),
                                                                    h.pat_bcol.as<int32_t>(), h.mass.as<double>(), w.t,
                                                                    0.0, w.mt);
-        dot(h, w, w.t, w.mt, nullptr, S_M, AFTER_NONE);
+        dot(h, w, w.t, w.mt, nullptr, S_M);
     }
-    if (h.obj_f) dot(h, w, h.obj_f, x, nullptr, S_F, AFTER_NONE);
+    if (h.obj_f) dot(h, w, h.obj_f, x, nullptr, S_F);
     PF_LAUNCH_CHECK();
 }
 
@@ -707,10 +736,10 @@ void objective_gradient(Handle &h, const Work &w, const double *x, double *g, in
         k_mass_apply<<<grid_for(h.n_nodes, BLOCK / SPMV_LANES), BLOCK, 0, h.stream>>>(h.n_nodes, h.brow_ptr.as<int32_t>(),
                                                                    h.pat_bcol.as<int32_t>(), h.mass.as<double>(), w.t,
                                                                    0.0, w.mt);
-        dot(h, w, w.t, w.mt, nullptr, S_M, AFTER_NONE);
+        dot(h, w, w.t, w.mt, nullptr, S_M);
         mt = w.mt;
     }
-    if (h.obj_f) dot(h, w, h.obj_f, x, nullptr, S_F, AFTER_NONE);
+    if (h.obj_f) dot(h, w, h.obj_f, x, nullptr, S_F);
     if (mt || h.obj_f || h.obj_w != 1.0)
         k_combine_gradient<<<grid_for(h.n_dofs), BLOCK, 0, h.stream>>>(g, h.obj_w, mt, h.obj_f, h.n_dofs);
     PF_LAUNCH_CHECK();
@@ -858,7 +887,7 @@ void newton_solve(Handle &h, double *x, const uint8_t *fixed, const pfgpu_newton
         h.op_valid = false; // a new iterate: the CG operator is rebuilt at x
         // energy and gradient at x; the reduced gradient norm
         objective_gradient(h, w, x, w.g, S_E0);
-        dot(h, w, w.g, w.g, fixed, S_B2, AFTER_NONE);
+        dot(h, w, w.g, w.g, fixed, S_B2);
         const double gn = std::sqrt(read_scalar(h, w, S_B2));
         const double e0 = objective_value(h, w, S_E0);
         rep.energy = e0;
@@ -897,7 +926,7 @@ void newton_solve(Handle &h, double *x, const uint8_t *fixed, const pfgpu_newton
         else
             rep.cg_stops_tolerance++;
         // direction in w.y; g.d for the Armijo condition
-        dot(h, w, w.g, w.y, fixed, S_GD, AFTER_NONE);
+        dot(h, w, w.g, w.y, fixed, S_GD);
         double gd = read_scalar(h, w, S_GD);
         const double *dir = w.y;
         if (!(gd < 0.0)) {
@@ -942,7 +971,7 @@ void newton_solve(Handle &h, double *x, const uint8_t *fixed, const pfgpu_newton
             // g is not positive
             k_neg_free<<<gr, BLOCK, 0, h.stream>>>(w.y, w.g, fixed, h.n_dofs);
             hvp_any(h, x, w.y, w.q);
-            dot(h, w, w.y, w.q, fixed, S_GD, AFTER_NONE);
+            dot(h, w, w.y, w.q, fixed, S_GD);
             const double c = read_scalar(h, w, S_GD);
             const double a0 = c > 0.0 ? gn * gn / c : 1.0 / gn;
             accepted = search(w.y, -gn * gn, a0);
@@ -957,7 +986,7 @@ void newton_solve(Handle &h, double *x, const uint8_t *fixed, const pfgpu_newton
     }
     // final state
     objective_gradient(h, w, x, w.g, S_E0);
-    dot(h, w, w.g, w.g, fixed, S_B2, AFTER_NONE);
+    dot(h, w, w.g, w.g, fixed, S_B2);
     rep.grad_norm = std::sqrt(read_scalar(h, w, S_B2));
     rep.energy = objective_value(h, w, S_E0);
     rep.converged = rep.grad_norm <= prm.grad_norm || rep.grad_norm <= prm.relative_grad_norm * gn0;
@@ -1186,40 +1215,48 @@ namespace {
 
 constexpr int SEG_CHUNK = 4095; // dofs: whole nodes
 
-// per-problem PCG state (device), one entry per problem
+// per-problem PCG state (device), one entry per problem; old, stop: r.z and the
+// done flag of the running iteration as the update kernel leaves them for the
+// direction kernel, which writes rz and done
 struct SegState {
-    double *rr, *rz, *b2, *alpha, *beta, *done, *iters, *active;
+    double *rr, *rz, *b2, *alpha, *old, *stop, *done, *iters, *active;
 };
 
-__device__ double block_sum(double v, double *sh)
-{
-    const int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int w = BLOCK / 2; w > 0; w >>= 1) {
-        if (t < w) sh[t] += sh[t + w];
-        __syncthreads();
-    }
-    return sh[0];
-}
-
 // part[c] = sum over chunk c's free dofs of a b; with done, 0 for the chunks
-// of finished problems (cs: chunk -> problem), whose partials nobody reads
+// of finished problems (cs: chunk -> problem), whose partials nobody reads, and
+// *active is cleared.  A thread's products are all loaded before they are
+// added: a chunk is one workgroup's work, and few chunks leave the latency of
+// its loads uncovered.
 __global__ __launch_bounds__(BLOCK) void k_chunk_dot(const double *__restrict__ a, const double *__restrict__ b,
                                                      const uint8_t *__restrict__ mask, const int32_t *__restrict__ cb,
                                                      double *__restrict__ part, const int32_t *__restrict__ cs = nullptr,
-                                                     const double *__restrict__ done = nullptr)
+                                                     const double *__restrict__ done = nullptr,
+                                                     double *__restrict__ active = nullptr)
 {
+    constexpr int N = (SEG_CHUNK + BLOCK - 1) / BLOCK;
     __shared__ double sh[BLOCK];
     const int c = blockIdx.x;
+    if (active && c == 0 && threadIdx.x == 0) *active = 0.0;
     if (done && done[cs[c]] != 0.0) { // uniform over the workgroup
         if (threadIdx.x == 0) part[c] = 0.0;
         return;
     }
+    const int i0 = cb[c] + threadIdx.x, end = cb[c + 1];
+    double av[N], bv[N];
+    bool use[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int i = i0 + k * BLOCK;
+        const bool in = i < end;
+        av[k] = in ? a[i] : 0.0;
+        bv[k] = in ? b[i] : 0.0;
+        use[k] = in && !(mask && mask[i]);
+    }
     double acc = 0;
-    for (int i = cb[c] + threadIdx.x; i < cb[c + 1]; i += BLOCK)
-        if (!mask || !mask[i]) acc = fma(a[i], b[i], acc);
-    const double v = block_sum(acc, sh);
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        if (use[k]) acc = fma(av[k], bv[k], acc);
+    const double v = block_reduce(acc, sh);
     if (threadIdx.x == 0) part[c] = v;
 }
 
@@ -1257,12 +1294,12 @@ __global__ __launch_bounds__(SEGW) void k_seg_total(const double *__restrict__ p
     }
 }
 
-// PCG start over chunk c's nodes: y = 0, r = b on free dofs, z = P r, p = z;
+// PCG start over chunk c's nodes: y = 0, r = b on free dofs, p = z = P r;
 // partials of r.z and r.r
 __global__ __launch_bounds__(BLOCK) void k_chunk_pcg_start(const double *__restrict__ b, const uint8_t *__restrict__ mask,
                                                            const float *__restrict__ pinv, const int32_t *__restrict__ cb,
                                                            double *__restrict__ y, double *__restrict__ r,
-                                                           double *__restrict__ z, double *__restrict__ p,
+                                                           double *__restrict__ p,
                                                            double *__restrict__ part_rz, double *__restrict__ part_rr)
 {
     __shared__ double sh[BLOCK];
@@ -1278,13 +1315,12 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_pcg_start(const double *__restr
         for (int d = 0; d < 3; ++d) {
             y[o + d] = 0.0;
             r[o + d] = ri[d];
-            z[o + d] = zi[d];
             p[o + d] = zi[d];
             rz = fma(ri[d], zi[d], rz);
             rr = fma(ri[d], ri[d], rr);
         }
     }
-    const double a = block_sum(rz, sh), e = block_sum(rr, sh);
+    const double a = block_reduce(rz, sh), e = block_reduce(rr, sh);
     if (threadIdx.x == 0) {
         part_rz[c] = a;
         part_rr[c] = e;
@@ -1313,120 +1349,137 @@ __global__ __launch_bounds__(SEGW) void k_seg_cg_start(const double *__restrict_
     if (threadIdx.x == 0) *st.active = a;
 }
 
-// Per-iteration scalar kernels: one wavefront per problem over a grid of
-// seg_grid(nseg) workgroups (problem s on wavefront s mod 16 of workgroup
-// s / 16); the count of problems still iterating is added into *active by
-// each workgroup (exact: a sum of small integers in FP64), which k_seg_alpha
-// clears first.
-inline unsigned seg_grid(int nseg) { return unsigned(std::max(1, (nseg + SEGW / WAVE - 1) / (SEGW / WAVE))); }
+// nodes of a chunk per thread: all of their loads are issued before the first use
+constexpr int SEG_NODES = (SEG_CHUNK / 3 + BLOCK - 1) / BLOCK;
 
-// alpha = r.z / p.Hp per problem; a non-positive curvature ends that problem
-__global__ __launch_bounds__(SEGW) void k_seg_alpha(const double *__restrict__ part, const int32_t *__restrict__ scp,
-                                                    int nseg, SegState st)
-{
-    if (blockIdx.x == 0 && threadIdx.x == 0) *st.active = 0.0;
-    for (int s = int(blockIdx.x * (SEGW / WAVE) + threadIdx.x / WAVE); s < nseg; s += int(gridDim.x) * (SEGW / WAVE)) {
-        const double pq = seg_total(part, scp, s);
-        if (threadIdx.x % WAVE != 0) continue;
-        if (st.done[s] != 0.0) {
-            st.alpha[s] = 0.0;
-        } else if (!(pq > 0.0)) {
-            st.alpha[s] = 0.0;
-            st.done[s] = 1.0;
-        } else {
-            st.alpha[s] = st.rz[s] / pq;
-        }
-    }
-}
-
-// y += alpha p, r -= alpha q on free dofs, z = P r over chunk c's nodes;
-// partials of the new r.z and r.r.  The chunks of a finished problem (done)
-// keep their vectors and give zero partials, which nobody reads.
-__global__ __launch_bounds__(BLOCK) void k_chunk_pcg_update(double *__restrict__ y, double *__restrict__ r,
-                                                            double *__restrict__ z, const double *__restrict__ p,
-                                                            const double *__restrict__ q, const uint8_t *__restrict__ mask,
-                                                            const float *__restrict__ pinv, const int32_t *__restrict__ cb,
-                                                            const int32_t *__restrict__ cs, const double *__restrict__ alpha,
-                                                            const double *__restrict__ done, double *__restrict__ part_rz,
-                                                            double *__restrict__ part_rr)
+// alpha = r.z / p.Hp of the chunk's problem (a non-positive curvature ends that
+// problem), then r -= alpha q on free dofs over the chunk's nodes; partials of
+// r.z, z = P r, and r.r.  Every wavefront adds the problem's p.Hp partials
+// itself, in the same order (instead of a launch of its own before this one),
+// and the problem's first chunk keeps the state.  The chunks of a finished
+// problem keep their vectors and give zero partials, which nobody reads.  16
+// problems of 4,374 tets: an iteration of seven kernels and 52 us became one of
+// five and 40, with a thread's loads issued together (dot 10.6 -> 7.7 us).
+__global__ __launch_bounds__(BLOCK) void k_chunk_pcg_update(double *__restrict__ r, const double *__restrict__ q,
+                                                            const uint8_t *__restrict__ mask, const float *__restrict__ pinv,
+                                                            const int32_t *__restrict__ cb, const int32_t *__restrict__ cs,
+                                                            const int32_t *__restrict__ scp,
+                                                            const double *__restrict__ part_pq, double *__restrict__ part_rz,
+                                                            double *__restrict__ part_rr, SegState st)
 {
     __shared__ double sh[BLOCK];
-    const int c = blockIdx.x;
-    if (done[cs[c]] != 0.0) { // uniform over the workgroup
+    const int c = blockIdx.x, s = cs[c];
+    const double pq = seg_total(part_pq, scp, s), old = st.rz[s];
+    const bool run = st.done[s] == 0.0 && pq > 0.0; // uniform over the problem's workgroups
+    const double a = run ? old / pq : 0.0;
+    if (threadIdx.x == 0 && c == scp[s]) {
+        st.alpha[s] = a;
+        st.old[s] = old;
+        st.stop[s] = run ? 0.0 : 1.0;
+    }
+    if (!run) {
         if (threadIdx.x == 0) part_rz[c] = part_rr[c] = 0.0;
         return;
     }
-    const double a = alpha[cs[c]];
-    double rz = 0, rr = 0;
-    for (int i = cb[c] / 3 + threadIdx.x; i < cb[c + 1] / 3; i += BLOCK) {
-        const int64_t o = 3 * int64_t(i);
-        // every load of the node first, then the masked update
-        double ri[3], zi[3], pi[3], qi[3], yi[3];
-        bool upd[3];
+    const int i0 = cb[c] / 3 + int(threadIdx.x), end = cb[c + 1] / 3;
+    double rv[SEG_NODES][3], qv[SEG_NODES][3];
+    bool upd[SEG_NODES][3];
+#pragma unroll
+    for (int k = 0; k < SEG_NODES; ++k) {
+        const int i = i0 + k * BLOCK;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            ri[d] = r[o + d];
-            pi[d] = p[o + d];
-            qi[d] = q[o + d];
-            yi[d] = y[o + d];
-            upd[d] = a != 0.0 && !mask[o + d];
+            const bool in = i < end;
+            const int64_t o = 3 * int64_t(i) + d;
+            rv[k][d] = in ? r[o] : 0.0;
+            qv[k][d] = in ? q[o] : 0.0;
+            upd[k][d] = in && a != 0.0 && !mask[o];
         }
+    }
+    double rz = 0, rr = 0;
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-            if (upd[d]) {
-                y[o + d] = fma(a, pi[d], yi[d]);
-                ri[d] = fma(-a, qi[d], ri[d]);
+    for (int k = 0; k < SEG_NODES; ++k) {
+        const int i = i0 + k * BLOCK;
+        if (i >= end) continue;
+        const int64_t o = 3 * int64_t(i);
+        double ri[3], zi[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            ri[d] = rv[k][d];
+            if (upd[k][d]) {
+                ri[d] = fma(-a, qv[k][d], ri[d]);
                 r[o + d] = ri[d];
             }
+        }
         precondition(pinv, i, ri, zi);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            z[o + d] = zi[d];
             rz = fma(ri[d], zi[d], rz);
             rr = fma(ri[d], ri[d], rr);
         }
     }
-    const double e = block_sum(rz, sh), f = block_sum(rr, sh);
+    const double e = block_reduce(rz, sh), f = block_reduce(rr, sh);
     if (threadIdx.x == 0) {
         part_rz[c] = e;
         part_rr[c] = f;
     }
 }
 
-// beta = r'.z' / r.z per problem; convergence at ||r|| <= tol ||b||
-__global__ __launch_bounds__(SEGW) void k_seg_beta(const double *__restrict__ part_rz, const double *__restrict__ part_rr,
-                                                   const int32_t *__restrict__ scp, int nseg, double tol2, SegState st)
-{
-    __shared__ double sh[SEGW / WAVE];
-    double act = 0;
-    for (int s = int(blockIdx.x * (SEGW / WAVE) + threadIdx.x / WAVE); s < nseg; s += int(gridDim.x) * (SEGW / WAVE)) {
-        const double rn = seg_total(part_rr, scp, s), zn = seg_total(part_rz, scp, s);
-        if (threadIdx.x % WAVE != 0) continue;
-        if (!isfinite(rn) || !isfinite(zn)) act += __builtin_nan(""); // reported to the host as a failed solve
-        if (st.done[s] == 0.0) {
-            st.iters[s] += 1.0;
-            st.beta[s] = st.rz[s] > 0.0 ? zn / st.rz[s] : 0.0;
-            st.rr[s] = rn;
-            st.rz[s] = zn;
-            if (rn <= tol2 * st.b2[s]) st.done[s] = 1.0;
-        } else {
-            st.beta[s] = 0.0;
-        }
-        act += st.done[s] == 0.0 ? 1.0 : 0.0;
-    }
-    const double a = wave_values_sum(act, sh);
-    if (threadIdx.x == 0) atomicAdd(st.active, a);
-}
-
-// p = z + beta p for the problems still iterating
-__global__ __launch_bounds__(BLOCK) void k_chunk_cg_direction(double *__restrict__ p, const double *__restrict__ z,
-                                                              const int32_t *__restrict__ cb, const int32_t *__restrict__ cs,
-                                                              const double *__restrict__ beta, const double *__restrict__ done)
+// beta = r'.z' / r.z of the chunk's problem and its convergence at
+// ||r|| <= tol ||b||, then y += alpha p on free dofs and, where the problem goes
+// on, p = z + beta p, z = P r formed again.  The partials are added as in
+// k_chunk_pcg_update; a problem's first chunk keeps its state and adds it to the
+// problems still iterating (exact: small integers in FP64), or NaN for a
+// non-finite residual, reported to the host as a failed solve.
+constexpr int SEG_DIRECTION = 1024; // threads: nothing here is summed in order
+__global__ __launch_bounds__(SEG_DIRECTION) void k_chunk_cg_direction(double *__restrict__ y, double *__restrict__ p,
+                                                                      const double *__restrict__ r,
+                                                                      const uint8_t *__restrict__ mask,
+                                                                      const float *__restrict__ pinv,
+                                                                      const int32_t *__restrict__ cb,
+                                                                      const int32_t *__restrict__ cs,
+                                                                      const int32_t *__restrict__ scp,
+                                                                      const double *__restrict__ part_rz,
+                                                                      const double *__restrict__ part_rr, double tol2,
+                                                                      SegState st)
 {
     const int c = blockIdx.x, s = cs[c];
-    if (done[s] != 0.0) return;
-    const double b = beta[s];
-    for (int i = cb[c] + threadIdx.x; i < cb[c + 1]; i += BLOCK) p[i] = fma(b, p[i], z[i]);
+    const bool first = threadIdx.x == 0 && c == scp[s];
+    if (st.stop[s] != 0.0) { // uniform over the problem's workgroups
+        if (first) st.done[s] = 1.0;
+        return;
+    }
+    const double zn = seg_total(part_rz, scp, s), rn = seg_total(part_rr, scp, s), old = st.old[s], a = st.alpha[s];
+    const double beta = old > 0.0 ? zn / old : 0.0;
+    const bool converged = rn <= tol2 * st.b2[s];
+    if (first) {
+        if (!isfinite(rn) || !isfinite(zn)) atomicAdd(st.active, __builtin_nan(""));
+        st.iters[s] += 1.0;
+        st.rr[s] = rn;
+        st.rz[s] = zn;
+        if (converged)
+            st.done[s] = 1.0;
+        else
+            atomicAdd(st.active, 1.0);
+    }
+    for (int i = cb[c] / 3 + int(threadIdx.x); i < cb[c + 1] / 3; i += SEG_DIRECTION) {
+        const int64_t o = 3 * int64_t(i);
+        double ri[3], zi[3], pi[3], yi[3];
+        bool upd[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            ri[d] = r[o + d];
+            pi[d] = p[o + d];
+            yi[d] = y[o + d];
+            upd[d] = a != 0.0 && !mask[o + d];
+        }
+        precondition(pinv, i, ri, zi);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (upd[d]) y[o + d] = fma(a, pi[d], yi[d]);
+            if (!converged) p[o + d] = fma(beta, pi[d], zi[d]);
+        }
+    }
 }
 
 // out[s] = sum of v[off[s] .. off[s+1]) (one block per segment, fixed order)
@@ -1437,7 +1490,7 @@ __global__ __launch_bounds__(BLOCK) void k_seg_sum(const double *__restrict__ v,
     const int sgm = blockIdx.x;
     double a = 0;
     for (int i = off[sgm] + threadIdx.x; i < off[sgm + 1]; i += BLOCK) a += v[i];
-    const double tot = block_sum(a, sh);
+    const double tot = block_reduce(a, sh);
     if (threadIdx.x == 0) out[sgm] = tot;
 }
 
@@ -1469,7 +1522,7 @@ __global__ __launch_bounds__(BLOCK) void k_seg_steepest(double *__restrict__ d, 
 
 // chunks of at most SEG_CHUNK dofs inside each problem's dof range
 struct SegChunks {
-    DevBuf cb, cs, scp, part, part2;
+    DevBuf cb, cs, scp, part, part2, part3;
     int n = 0;
 };
 
@@ -1491,34 +1544,32 @@ SegChunks seg_chunks(const int32_t *no, int nseg, hipStream_t st)
     c.scp = upload(scp, st);
     c.part = DevBuf{sizeof(double) * size_t(c.n)};
     c.part2 = DevBuf{sizeof(double) * size_t(c.n)};
+    c.part3 = DevBuf{sizeof(double) * size_t(c.n)};
     return c;
 }
 
 // PCG start of every active problem (a fixed kernel sequence)
 void seg_cg_start(Handle &h, const Work &w, const uint8_t *mask, const SegChunks &ch, int nseg, const SegState &st)
 {
-    k_chunk_pcg_start<<<ch.n, BLOCK, 0, h.stream>>>(w.d, mask, precond(h), ch.cb.as<int32_t>(), w.y, w.r, w.z, w.p,
+    k_chunk_pcg_start<<<ch.n, BLOCK, 0, h.stream>>>(w.d, mask, precond(h), ch.cb.as<int32_t>(), w.y, w.r, w.p,
                                                     ch.part.as<double>(), ch.part2.as<double>());
     k_seg_cg_start<<<1, SEGW, 0, h.stream>>>(ch.part.as<double>(), ch.part2.as<double>(), ch.scp.as<int32_t>(), nseg, st);
     PF_LAUNCH_CHECK();
 }
 
 // One PCG iteration on every active problem at once (a fixed kernel sequence).
-void seg_cg_iteration(Handle &h, const Work &w, const double *x, const uint8_t *mask, const SegChunks &ch, int nseg,
-                      double tol2, const SegState &st)
+void seg_cg_iteration(Handle &h, const Work &w, const double *x, const uint8_t *mask, const SegChunks &ch, double tol2,
+                      const SegState &st)
 {
     hvp_any(h, x, w.p, w.q);
     k_chunk_dot<<<ch.n, BLOCK, 0, h.stream>>>(w.p, w.q, mask, ch.cb.as<int32_t>(), ch.part.as<double>(),
-                                              ch.cs.as<int32_t>(), st.done);
-    k_seg_alpha<<<seg_grid(nseg), SEGW, 0, h.stream>>>(ch.part.as<double>(), ch.scp.as<int32_t>(), nseg, st);
-    k_chunk_pcg_update<<<ch.n, BLOCK, 0, h.stream>>>(w.y, w.r, w.z, w.p, w.q, mask, precond(h), ch.cb.as<int32_t>(),
-                                                     ch.cs.as<int32_t>(), st.alpha, st.done, ch.part.as<double>(),
-                                                     ch.part2.as<double>());
-    k_seg_beta<<<seg_grid(nseg), SEGW, 0, h.stream>>>(ch.part.as<double>(), ch.part2.as<double>(), ch.scp.as<int32_t>(),
-                                                      nseg, tol2,
-                                          st);
-    k_chunk_cg_direction<<<ch.n, BLOCK, 0, h.stream>>>(w.p, w.z, ch.cb.as<int32_t>(), ch.cs.as<int32_t>(), st.beta,
-                                                       st.done);
+                                              ch.cs.as<int32_t>(), st.done, st.active);
+    k_chunk_pcg_update<<<ch.n, BLOCK, 0, h.stream>>>(w.r, w.q, mask, precond(h), ch.cb.as<int32_t>(), ch.cs.as<int32_t>(),
+                                                     ch.scp.as<int32_t>(), ch.part.as<double>(), ch.part2.as<double>(),
+                                                     ch.part3.as<double>(), st);
+    k_chunk_cg_direction<<<ch.n, SEG_DIRECTION, 0, h.stream>>>(w.y, w.p, w.r, mask, precond(h), ch.cb.as<int32_t>(),
+                                                               ch.cs.as<int32_t>(), ch.scp.as<int32_t>(),
+                                                               ch.part2.as<double>(), ch.part3.as<double>(), tol2, st);
     PF_LAUNCH_CHECK();
 }
 
@@ -1543,12 +1594,12 @@ void newton_solve_batch(Handle &h, double *x, const uint8_t *fixed, int nseg, co
     DevBuf d_eseg = upload(eseg_of, h.stream);
     const SegChunks ch = seg_chunks(no_h, nseg, h.stream);
     const size_t ns = size_t(nseg);
-    // doubles: energy, gradient norm, g.d, step (4 ns), PCG state (7 ns + 1); then two byte flags per problem
-    DevBuf scal{sizeof(double) * (11 * ns + 1) + 2 * ns}, pe{sizeof(double) * size_t(E)}, mask{size_t(n)};
+    // doubles: energy, gradient norm, g.d, step (4 ns), PCG state (8 ns + 1); then two byte flags per problem
+    DevBuf scal{sizeof(double) * (12 * ns + 1) + 2 * ns}, pe{sizeof(double) * size_t(E)}, mask{size_t(n)};
     double *s_e = scal.as<double>(), *s_g = s_e + ns, *s_gd = s_g + ns, *s_a = s_gd + ns;
-    const SegState st{s_a + ns,     s_a + 2 * ns, s_a + 3 * ns, s_a + 4 * ns,
-                      s_a + 5 * ns, s_a + 6 * ns, s_a + 7 * ns, s_a + 8 * ns};
-    uint8_t *frozen = reinterpret_cast<uint8_t *>(s_a + 8 * ns + 1), *flag = frozen + ns;
+    const SegState st{s_a + ns,     s_a + 2 * ns, s_a + 3 * ns, s_a + 4 * ns, s_a + 5 * ns,
+                      s_a + 6 * ns, s_a + 7 * ns, s_a + 8 * ns, s_a + 9 * ns};
+    uint8_t *frozen = reinterpret_cast<uint8_t *>(s_a + 9 * ns + 1), *flag = frozen + ns;
     std::vector<double> e0(ns), e1(ns), gn(ns), gn0(ns), gd(ns), alpha(ns), it_cg(ns);
     std::vector<uint8_t> fr(ns, 0), fl(ns, 0);
     std::vector<pfgpu_newton_report> rep(ns);
@@ -1607,12 +1658,12 @@ void newton_solve_batch(Handle &h, double *x, const uint8_t *fixed, int nseg, co
         }
         if (prm.use_graph && !graph) {
             // an eager iteration sizes every scratch buffer; then restart and capture
-            seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, nseg, tol2, st);
+            seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, tol2, st);
             seg_cg_start(h, w, mask.as<uint8_t>(), ch, nseg, st);
             hipGraph_t g = nullptr;
             PF_HIP(hipStreamBeginCapture(h.stream, hipStreamCaptureModeThreadLocal));
             try {
-                for (int k = 0; k < CHECK; ++k) seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, nseg, tol2, st);
+                for (int k = 0; k < CHECK; ++k) seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, tol2, st);
             } catch (...) {
                 (void)hipStreamEndCapture(h.stream, &g);
                 if (g) (void)hipGraphDestroy(g);
@@ -1634,7 +1685,7 @@ void newton_solve_batch(Handle &h, double *x, const uint8_t *fixed, int nseg, co
             if (graph && k == CHECK)
                 PF_HIP(hipGraphLaunch(graph, h.stream));
             else
-                for (int j = 0; j < k; ++j) seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, nseg, tol2, st);
+                for (int j = 0; j < k; ++j) seg_cg_iteration(h, w, x, mask.as<uint8_t>(), ch, tol2, st);
             it += k;
             PF_HIP(hipMemcpyAsync(act.data(), st.active, sizeof(double), hipMemcpyDeviceToHost, h.stream));
             PF_HIP(hipStreamSynchronize(h.stream));
