@@ -32,6 +32,10 @@ struct pfgpu_handle {
     // plan of the segmented node-row gather (chunks, padded slots, row metadata)
     pfgpu::DevBuf row_chunk, row_slot, row_meta;
     int n_row_chunks = 0;
+    // chunks of the vertex gather (shape derivative): (first vertex, first
+    // incidence); -1: a vertex lies in more elements than a chunk holds
+    pfgpu::DevBuf vert_chunk;
+    int n_vert_chunks = 0;
     // factored Hessian (PFGPU_PATH_FACTORED): per-element factor records
     pfgpu::DevBuf fac_rec;
     int n_cu = 0; // compute units of the device (queried on first use)
