@@ -131,8 +131,8 @@ const double *stage(pfgpu_handle &h, DevBuf &buf, const double *host, size_t n)
 
 void fetch(pfgpu_handle &h, void *host, const void *dev, size_t bytes)
 {
-    PF_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, h.stream));
-    PF_HIP(hipStreamSynchronize(h.stream));
+    const HostCopy item{host, dev, bytes};
+    copy_to_host(h, &item, 1);
 }
 
 void gradient_dev(pfgpu_handle &h, const double *x, double *g, double *energy)
@@ -168,17 +168,19 @@ void hvp_dev(pfgpu_handle &h, const double *x, const double *v, double *y)
         plain_hvp(h, x, v, y);
 }
 
-void check_finite(pfgpu_handle &h, const void *dev, int64_t n, bool is_float, const char *what)
+[[noreturn]] void fail_nonfinite(const char *what)
 {
-    if (!all_finite(h, dev, n, is_float))
-        fail(PFGPU_ERR_INVALID_STATE, std::string(what) + " has non-finite entries (inverted element?)");
+    fail(PFGPU_ERR_INVALID_STATE, std::string(what) + " has non-finite entries (inverted element?)");
 }
 
 } // namespace
 
+pfgpu_handle::pfgpu_handle() { pfgpu::host_copy_handles(1); }
+
 pfgpu_handle::~pfgpu_handle()
 {
     pfgpu::solver_release(*this);
+    pfgpu::host_copy_handles(-1);
     if (own_stream) (void)hipStreamDestroy(own_stream);
 }
 
@@ -607,8 +609,10 @@ pfgpu_status pfgpu_hessian_values(pfgpu_handle *h, const double *x, int32_t proj
             plain_hessian(*h, dx, h->h_vals.get(), true); // the projection runs on the element tiles of the plain path
         else
             egh_dev(*h, dx, nullptr, nullptr, h->h_vals.get());
-        check_finite(*h, h->h_vals.get(), h->pat.nnz, h->precision == PFGPU_MIXED, "Hessian");
-        fetch(*h, values, h->h_vals.get(), bytes);
+        int bad = 0;
+        const int *flag = count_nonfinite(*h, h->h_vals.get(), h->pat.nnz, h->precision == PFGPU_MIXED);
+        const HostCopy items[2] = {{&bad, flag, sizeof(bad)}, {values, h->h_vals.get(), bytes}};
+        if (!copy_to_host(*h, items, 2, &bad)) fail_nonfinite("Hessian");
     });
 }
 
@@ -634,14 +638,19 @@ pfgpu_status pfgpu_energy_gradient_hessian(pfgpu_handle *h, const double *x, dou
             dv = h->h_vals.get();
         }
         egh_dev(*h, dx, de, dg, dv);
-        if (energy) fetch(*h, energy, de, sizeof(double));
-        if (g) fetch(*h, g, dg, sizeof(double) * size_t(h->n_dofs));
-        if (values) fetch(*h, values, dv, bytes);
+        int bad = 0;
+        HostCopy items[4];
+        int n = 0;
+        if (values) items[n++] = {&bad, count_nonfinite(*h, dv, h->pat.nnz, h->precision == PFGPU_MIXED), sizeof(bad)};
+        if (energy) items[n++] = {energy, de, sizeof(double)};
+        if (g) items[n++] = {g, dg, sizeof(double) * size_t(h->n_dofs)};
+        if (values) items[n++] = {values, dv, bytes};
+        copy_to_host(*h, items, n);
         if (energy && !std::isfinite(*energy)) fail(PFGPU_ERR_INVALID_STATE, "energy is not finite (inverted element?)");
         if (g)
             for (int i = 0; i < h->n_dofs; ++i)
                 if (!std::isfinite(g[i])) fail(PFGPU_ERR_INVALID_STATE, "gradient is not finite (inverted element?)");
-        if (values) check_finite(*h, dv, h->pat.nnz, h->precision == PFGPU_MIXED, "Hessian");
+        if (bad) fail_nonfinite("Hessian");
     });
 }
 

@@ -102,6 +102,7 @@ struct pfgpu_handle {
     std::vector<std::unique_ptr<pfgpu_handle>> groups;
     std::vector<int32_t> batch_perm;     // caller's problem index of each problem, in group order
     std::vector<int32_t> batch_eo, batch_no; // element / node offsets of the problems, group order
+    pfgpu_handle();
     ~pfgpu_handle();
 
     size_t value_size() const { return precision == PFGPU_MIXED ? sizeof(float) : sizeof(double); }
@@ -188,6 +189,18 @@ void solver_release(Handle &h);
 // ---- misc kernels (reduce.hip) ----------------------------------------
 void build_device_pattern(Handle &h);
 // returns true when every value in the device array is finite
+// *flag (device) becomes 1 where v has a non-finite entry, else 0
+int *count_nonfinite(Handle &h, const void *dev, int64_t n, bool is_float);
 bool all_finite(Handle &h, const void *dev, int64_t n, bool is_float);
+// device results into host arrays (host_copy.cpp), complete on return; with stop,
+// one of the items' hosts, false as soon as it arrives non-zero (later items are
+// then not written)
+struct HostCopy {
+    void *host;
+    const void *dev;
+    size_t bytes;
+};
+bool copy_to_host(Handle &h, const HostCopy *items, int n_items, const int *stop = nullptr);
+void host_copy_handles(int delta); // the handles alive, which hold the pinned rings
 
 } // namespace pfgpu

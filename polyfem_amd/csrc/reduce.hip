@@ -101,7 +101,7 @@ void sum_doubles(Handle &h, const double *in, int n, double *out)
     sum_doubles_into(h, in, n, out, h.sum_part.as<double>());
 }
 
-bool all_finite(Handle &h, const void *dev, int64_t n, bool is_float)
+int *count_nonfinite(Handle &h, const void *dev, int64_t n, bool is_float)
 {
     h.red_out.reserve(sizeof(int) * 4);
     int *flag = h.red_out.as<int>();
@@ -112,6 +112,12 @@ bool all_finite(Handle &h, const void *dev, int64_t n, bool is_float)
     else
         k_count_nonfinite<double><<<g, BLOCK, 0, h.stream>>>(static_cast<const double *>(dev), n, flag);
     PF_LAUNCH_CHECK();
+    return flag;
+}
+
+bool all_finite(Handle &h, const void *dev, int64_t n, bool is_float)
+{
+    const int *flag = count_nonfinite(h, dev, n, is_float);
     int host = 0;
     PF_HIP(hipMemcpyAsync(&host, flag, sizeof(int), hipMemcpyDeviceToHost, h.stream));
     PF_HIP(hipStreamSynchronize(h.stream));
