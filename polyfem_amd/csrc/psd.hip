@@ -244,22 +244,20 @@ constexpr int NS_FAST = 8, NS_POLISH = 10;
 constexpr float NS_A = 3.4445f, NS_B = -4.7750f, NS_C = 2.0315f;
 constexpr int NSS = 33; // row stride of a 32x32 matrix in LDS (conflict-free rows and columns)
 
-// P Q for 32x32 matrices in LDS, with v_mfma_f32_32x32x2f32 over k = 2s, 2s+1:
-// lane l supplies P[l % 32][2s + l / 32] and Q[2s + l / 32][l % 32]
-__device__ __forceinline__ floatx16 ns_mul(const float *P, const float *Q, int i0, int h)
+// A 32x32 matrix in the accumulator layout of v_mfma_f32_32x32x2f32: register r
+// of lane l holds row ns_row(r, l / 32) of column l % 32.
+__device__ __forceinline__ int ns_row(int r, int h) { return 8 * (r / 4) + 4 * h + (r % 4); }
+
+// P^T Q: step r of the product takes k = ns_row(r, 0) from the lower and
+// ns_row(r, 1) from the upper half of the lanes, so that both of its operands,
+// P[k][l % 32] and Q[k][l % 32], are the registers r of the accumulator layout.
+// Nothing goes through LDS.
+__device__ __forceinline__ floatx16 ns_mul(const floatx16 &P, const floatx16 &Q)
 {
     floatx16 acc = {};
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(P[i0 * NSS + 2 * s + h], Q[(2 * s + h) * NSS + i0], acc, 0, 0, 0);
+    for (int r = 0; r < 16; ++r) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(P[r], Q[r], acc, 0, 0, 0);
     return acc;
-}
-// row of accumulator r of lane half h (the column is l % 32)
-__device__ __forceinline__ int ns_row(int r, int h) { return 8 * (r / 4) + 4 * h + (r % 4); }
-__device__ __forceinline__ void ns_store(float *D, const floatx16 &v, int i0, int h)
-{
-#pragma unroll
-    for (int r = 0; r < 16; ++r) D[ns_row(r, h) * NSS + i0] = v[r];
 }
 
 // One wavefront per P2 element (30x30 padded to 32x32 with zeros, which
@@ -267,13 +265,16 @@ __device__ __forceinline__ void ns_store(float *D, const floatx16 &v, int i0, in
 // at rows and columns 0 and 16 of a block-diagonal 32x32, each scaled by its
 // own norm: polynomials in a block-diagonal X act on each block alone).  The
 // workgroup is the wavefront, so the barriers only order the LDS accesses of
-// its lanes.
+// its lanes.  The iterates stay in registers and feed the next product as they
+// lie; only X is transposed through LDS, once a step: X^T in its place would
+// let its rounding off symmetry grow 1.5 to 3.4 times a step between zero and
+// other eigenvalues, where powers of X itself keep it.  Bound by the matrix cores: 45 products of 16
+// instructions per wavefront; 16,380 P2 elements take 429 us (460 with every
+// operand read from LDS), 113 of the 150 TFLOP/s that a large FP32 product reaches.
 template <int ORDER> __global__ __launch_bounds__(64) void k_psd_ns(int n_elements, float *__restrict__ hloc)
 {
     constexpr int NB = ORDER == 1 ? 4 : 10, N = 3 * NB, NBLK = NB * (NB + 1) / 2, EPW = ORDER == 1 ? 2 : 1;
-    // A, the iterate X and a temporary W (X^2, then the polynomial factor):
-    // 12.7 KB, 12 wavefronts per CU
-    __shared__ float A[32 * NSS], X[32 * NSS], W[32 * NSS];
+    __shared__ float A[32 * NSS];
     const int lane = threadIdx.x, i0 = lane % 32, h = lane / 32;
     const int e0 = int(blockIdx.x) * EPW;
     if (e0 >= n_elements) return; // uniform over the workgroup
@@ -302,40 +303,48 @@ template <int ORDER> __global__ __launch_bounds__(64) void k_psd_ns(int n_elemen
         ss = wave_sum(ss);
         sc[k] = ss > 0.f ? 1.f / std::sqrt(ss) : 0.f; // a zero matrix stays zero
     }
-    for (int k = lane; k < 32 * NSS; k += 64) X[k] = A[k] * (EPW == 1 || k / NSS < 16 ? sc[0] : sc[EPW - 1]);
-    __syncthreads();
-    for (int it = 0; it < NS_FAST + NS_POLISH; ++it) {
-        const floatx16 x2 = ns_mul(X, X, i0, h);
-        floatx16 m;
-        if (it < NS_FAST) {
-            ns_store(W, x2, i0, h);
-            __syncthreads();
-            const floatx16 x4 = ns_mul(W, W, i0, h);
-            __syncthreads(); // every lane has read W
-#pragma unroll
-            for (int r = 0; r < 16; ++r) m[r] = fmaf(NS_C, x4[r], NS_B * x2[r]) + (ns_row(r, h) == i0 ? NS_A : 0.f);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) m[r] = -0.5f * x2[r] + (ns_row(r, h) == i0 ? 1.5f : 0.f);
-        }
-        ns_store(W, m, i0, h);
-        __syncthreads();
-        const floatx16 xn = ns_mul(X, W, i0, h);
-        __syncthreads(); // every lane has read X
-        ns_store(X, xn, i0, h);
-        __syncthreads();
-    }
-    const floatx16 ax = ns_mul(A, X, i0, h);
+    floatx16 a, x;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const int i = ns_row(r, h);
-        W[i * NSS + i0] = 0.5f * (A[i * NSS + i0] + ax[r]);
+        a[r] = A[ns_row(r, h) * NSS + i0];
+        x[r] = a[r] * (EPW == 1 || ns_row(r, h) < 16 ? sc[0] : sc[EPW - 1]);
     }
+    auto transposed = [&](const floatx16 &v) {
+        floatx16 t;
+        __syncthreads(); // A, or the previous transpose, is read
+#pragma unroll
+        for (int r = 0; r < 16; ++r) A[ns_row(r, h) * NSS + i0] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r] = A[i0 * NSS + ns_row(r, h)];
+        return t;
+    };
+    auto diagonal = [&](int r) { return ns_row(r, h) == i0; };
+#pragma unroll 1
+    for (int it = 0; it < NS_FAST; ++it) {
+        const floatx16 xt = transposed(x), x2 = ns_mul(xt, x), x4 = ns_mul(x2, x2);
+        floatx16 m;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) m[r] = fmaf(NS_C, x4[r], NS_B * x2[r]) + (diagonal(r) ? NS_A : 0.f);
+        x = ns_mul(xt, m);
+    }
+#pragma unroll 1
+    for (int it = 0; it < NS_POLISH; ++it) {
+        const floatx16 xt = transposed(x);
+        floatx16 m = ns_mul(xt, x);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) m[r] = -0.5f * m[r] + (diagonal(r) ? 1.5f : 0.f);
+        x = ns_mul(xt, m);
+    }
+    const floatx16 ax = ns_mul(a, x);
+    __syncthreads(); // the last transpose is read
+#pragma unroll
+    for (int r = 0; r < 16; ++r) A[ns_row(r, h) * NSS + i0] = 0.5f * (a[r] + ax[r]);
     __syncthreads();
     for (int i = lane; i < ne * NBLK * 9; i += 64) {
         const int k = i / (NBLK * 9), ii = i - k * NBLK * 9, s = ii / 9, j = ii % 9;
         const int r = 16 * k + 3 * bp.a[s] + j / 3, c = 16 * k + 3 * bp.b[s] + j % 3;
-        base(e0 + k)[int64_t(s) * 576 + j] = W[r * NSS + c];
+        base(e0 + k)[int64_t(s) * 576 + j] = A[r * NSS + c];
     }
 }
 
