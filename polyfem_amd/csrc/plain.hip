@@ -318,15 +318,24 @@ __global__ __launch_bounds__(HB) void k_hessian(DevMesh<T> m, const double *__re
 
 // local H(x) v; yloc[(e*NB + a)*3 + d].  One wavefront per workgroup: the
 // 64 elements' results are staged in LDS and stored as one contiguous run
-// (elements of finished problems compute and store nothing).  FP32 with the
-// NeoHookean, linear and SaintVenant tangents fits 168 VGPRs without spills:
-// three wavefronts per SIMD instead of two.
-template <typename T, int MAT> constexpr int hvp_waves()
+// (elements of finished problems compute and store nothing).
+//
+// Bound by the vector ALUs (57 % busy at 215,000 P2 tets FP32) and the latency
+// of the nodal loads.  Up to four points go through three phases, the field
+// gradients of x, the stress differentials, the contraction: no phase needs
+// both nodal vectors, all points and the result in registers, and FP32 P2 fits
+// 124 VGPRs where the loop over points takes 168: four wavefronts per SIMD
+// instead of three, and 3,357 wavefronts in one round (30.8 -> 27.6 us).  More
+// points (A alone would be 54 to 99 registers) and the corotational tangent,
+// whose own temporaries set the peak, keep the loop (11 points 24.3 us, in
+// phases 25.1; FixedCorotational FP64 41.8 and 42.4).
+template <int NQ, int MAT> constexpr bool hvp_phases() { return NQ <= 4 && MAT != MAT_FC; }
+template <typename T, int NQ, int MAT> constexpr int hvp_waves()
 {
-    return sizeof(T) == 4 && (MAT == MAT_NH || MAT == MAT_LE || MAT == MAT_SV) ? 3 : 1;
+    return sizeof(T) == 4 && (MAT == MAT_NH || MAT == MAT_LE || MAT == MAT_SV) ? (hvp_phases<NQ, MAT>() ? 4 : 3) : 1;
 }
 template <typename T, int ORDER, int NQ, int MAT>
-__global__ __launch_bounds__(64, (hvp_waves<T, MAT>())) void k_hvp(DevMesh<T> m, const double *__restrict__ x,
+__global__ __launch_bounds__(64, (hvp_waves<T, NQ, MAT>())) void k_hvp(DevMesh<T> m, const double *__restrict__ x,
                                                                    const double *__restrict__ v, T *__restrict__ yloc,
                                                                    SegSkip skip)
 {
@@ -338,22 +347,47 @@ __global__ __launch_bounds__(64, (hvp_waves<T, MAT>())) void k_hvp(DevMesh<T> m,
         load_geometry(m, e, el);
         gather(m, e, x, el.U);
         T V[NB][3];
-        gather(m, e, v, V);
         T y[NB][3];
+        if constexpr (hvp_phases<NQ, MAT>()) {
+            T A[NQ][9]; // field gradients, then stress differentials
 #pragma unroll
-        for (int a = 0; a < NB; ++a)
+            for (int q = 0; q < NQ; ++q) field_grad<T, ORDER, NQ>(q, el.U, el.jit, A[q]);
+            gather(m, e, v, V);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int d = 0; d < 3; ++d) y[a][d] = T(0);
+            for (int q = 0; q < NQ; ++q) {
+                Kin<T> k;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const T w = el.det * T(quad_weight(NQ, q));
-            Kin<T> k;
-            field_grad<T, ORDER, NQ>(q, el.U, el.jit, k.H);
-            if (MAT == MAT_NH || MAT == MAT_FC || MAT == MAT_MR) kinematics(k);
-            T Gv[9], A[9];
-            field_grad<T, ORDER, NQ>(q, V, el.jit, Gv);
-            dstress<T, MAT>(k, el.lam, el.mu, el.p3, Gv, A);
-            contract_add<T, ORDER, NQ>(q, A, el.jit, w, y);
+                for (int i = 0; i < 9; ++i) k.H[i] = A[q][i];
+                if (MAT == MAT_NH || MAT == MAT_FC || MAT == MAT_MR) kinematics(k);
+                T Gv[9];
+                field_grad<T, ORDER, NQ>(q, V, el.jit, Gv);
+                dstress<T, MAT>(k, el.lam, el.mu, el.p3, Gv, A[q]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int a = 0; a < NB; ++a)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) y[a][d] = T(0);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) contract_add<T, ORDER, NQ>(q, A[q], el.jit, el.det * T(quad_weight(NQ, q)), y);
+        } else {
+            gather(m, e, v, V);
+#pragma unroll
+            for (int a = 0; a < NB; ++a)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) y[a][d] = T(0);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const T w = el.det * T(quad_weight(NQ, q));
+                Kin<T> k;
+                field_grad<T, ORDER, NQ>(q, el.U, el.jit, k.H);
+                if (MAT == MAT_NH || MAT == MAT_FC || MAT == MAT_MR) kinematics(k);
+                T Gv[9], A[9];
+                field_grad<T, ORDER, NQ>(q, V, el.jit, Gv);
+                dstress<T, MAT>(k, el.lam, el.mu, el.p3, Gv, A);
+                contract_add<T, ORDER, NQ>(q, A, el.jit, w, y);
+            }
         }
 #pragma unroll
         for (int a = 0; a < NB; ++a)
