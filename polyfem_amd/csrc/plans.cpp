@@ -3,8 +3,8 @@
 // only, so that tests can build and check the plans on the CPU.
 #include <algorithm>
 #include <atomic>
-#include <functional>
 #include <thread>
+#include <utility>
 
 #include "plans.hpp"
 
@@ -235,12 +235,15 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
                bp[size_t(j) + 1] - bp[size_t(i)] <= WAVE_BLOCKS)
             ++j;
         WaveShape s;
+        int32_t hist[256] = {}; // blocks of every count
+        for (int32_t b = bp[size_t(i)]; b < bp[size_t(j)]; ++b) ++hist[count[size_t(b)]];
         while (true) {
-            cnt.assign(count.begin() + bp[size_t(i)], count.begin() + bp[size_t(j)]);
-            std::sort(cnt.begin(), cnt.end(), std::greater<int32_t>());
+            cnt.clear();
+            for (int c = cap; c >= 0; --c) cnt.insert(cnt.end(), size_t(hist[c]), c);
             s = wave_shape(cnt);
             if (j == i + 1 || (s.words <= word_cap && s.n_long <= 64)) break;
             --j;
+            for (int32_t b = bp[size_t(j)]; b < bp[size_t(j) + 1]; ++b) --hist[count[size_t(b)]];
         }
         if (s.n_long > 64) return false;
         WaveHead h{};
@@ -291,9 +294,11 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
                         list[size_t(next[size_t(k)]++)] = (u - h.unit0) * NB + b;
                     }
             }
-            for (int k = 0; k < nb; ++k) order[size_t(k)] = k;
-            std::stable_sort(order.begin(), order.end(),
-                             [&](int32_t x, int32_t y) { return count[size_t(B0 + x)] > count[size_t(B0 + y)]; });
+            // by descending count, the blocks of a count in their order
+            int32_t place[257] = {};
+            for (int k = 0; k < nb; ++k) ++place[count[size_t(B0 + k)]];
+            for (int c = cap, at = 0; c >= 0; --c) at += std::exchange(place[c], at);
+            for (int k = 0; k < nb; ++k) order[size_t(place[count[size_t(B0 + k)]]++)] = k;
             sorted.resize(size_t(nb));
             for (int j = 0; j < nb; ++j) sorted[size_t(j)] = count[size_t(B0 + order[size_t(j)])];
             const WaveShape s = wave_shape(sorted);
