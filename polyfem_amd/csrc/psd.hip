@@ -268,9 +268,10 @@ __device__ __forceinline__ floatx16 ns_mul(const floatx16 &P, const floatx16 &Q)
 // its lanes.  The iterates stay in registers and feed the next product as they
 // lie; only X is transposed through LDS, once a step: X^T in its place would
 // let its rounding off symmetry grow 1.5 to 3.4 times a step between zero and
-// other eigenvalues, where powers of X itself keep it.  Bound by the matrix cores: 45 products of 16
-// instructions per wavefront; 16,380 P2 elements take 429 us (460 with every
-// operand read from LDS), 113 of the 150 TFLOP/s that a large FP32 product reaches.
+// other eigenvalues, where powers of X itself keep it.  Bound by the matrix
+// cores: 45 products of 16 instructions per wavefront; 16,380 P2 elements take
+// 429 us (460 with every operand read from LDS), 113 of the 150 TFLOP/s that a
+// large FP32 product reaches.
 template <int ORDER> __global__ __launch_bounds__(64) void k_psd_ns(int n_elements, float *__restrict__ hloc)
 {
     constexpr int NB = ORDER == 1 ? 4 : 10, N = 3 * NB, NBLK = NB * (NB + 1) / 2, EPW = ORDER == 1 ? 2 : 1;
