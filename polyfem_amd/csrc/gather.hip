@@ -53,18 +53,6 @@ __device__ __forceinline__ double fma_t(double a, double b, double c) { return f
 
 constexpr int N_XCD = 8;
 
-// units per lane
-template <int ORDER, int NQ> constexpr int wave_rounds() { return ORDER == 1 && NQ == 1 ? 2 : 1; }
-// stage words of a chunk of several nodes (three workgroups of four in a CU's
-// LDS for FP32).  Fewer words leave lanes without a unit, more cost
-// wavefronts: P2 mixed 363 us, with 2,496 words 387; P1 mixed 151, with 1,600
-// words 160 and with 2,720 158; P1 FP64 (511,000 tets) 138, with 2,400 142.
-constexpr int wave_words(int order, int value_size) { return order == 2 ? 2528 : value_size == 4 ? 2400 : 1600; }
-// Wavefronts of a workgroup: they share the reference gradients alone.  P2
-// mixed 363 us, with two 376, with one 431 (its waves then are the limit of
-// workgroups per CU); of P2 FP64 one workgroup of eight fills the LDS.
-constexpr int wave_group(int order, int value_size) { return order == 2 && value_size == 8 ? 8 : 4; }
-
 // orders the LDS accesses of the wavefront's lanes (LDS serves a wavefront in order)
 __device__ __forceinline__ void wave_order()
 {
@@ -111,12 +99,13 @@ __global__ __launch_bounds__(64 * wave_group(ORDER, sizeof(T)), wave_waves(sizeo
     const uint32_t *__restrict__ desc, const uint32_t *__restrict__ long_desc, const T *__restrict__ rec,
     const T *__restrict__ gloc, T *__restrict__ values, double *__restrict__ grad)
 {
-    constexpr int NB = NLocal<ORDER>::value, R = fac_size(NQ), ROUNDS = wave_rounds<ORDER, NQ>(), AHEAD = wave_ahead(ORDER);
+    constexpr int NB = NLocal<ORDER>::value, R = fac_size(NQ), ROUNDS = wave_rounds(ORDER, NQ), AHEAD = wave_ahead(ORDER);
     constexpr int WAVES = wave_group(ORDER, sizeof(T));
     constexpr bool EDGES = ORDER == 2 && NQ == 4;
     constexpr int DW = NB / 2;
     // reference gradients of the lane's own node, [a][q] as (r0 r1 r2 0)
     __shared__ __align__(16) T srg[NB * NQ * 4];
+    static_assert(sizeof(srg) == wave_table(ORDER, NQ, sizeof(T)));
     extern __shared__ __align__(32) unsigned char stages[];
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     unsigned char *smem = stages + wave * words * int(sizeof(T)); // the wavefront's stage
@@ -470,14 +459,14 @@ __global__ __launch_bounds__(BLOCK) void k_zero_nodes(int n, const int32_t *__re
 } // namespace
 
 // the wavefront plan of the handle; false when a node has too many incident
-// elements for one chunk (the row-unit gather then serves the handle)
+// elements for one chunk, or blocks for a stage that the workgroup's LDS holds
+// (the row-unit gather then serves the handle)
 bool wave_plan_ready(Handle &h)
 {
     if (h.wave_plan.state == 0) {
-        const bool p1 = h.order == 1 && h.n_quad == 1;
         WavePlanHost w;
         if (9 * h.pat.n_blocks >= (int64_t(1) << 31) ||
-            !make_wave_plan(h.pat, h.n_local, h.h_elem_nodes.data(), p1 ? 2 : 1, wave_words(h.order, int(h.value_size())), int(h.value_size()), w)) {
+            !plan_wave_gather(h.pat, h.order, h.n_quad, h.h_elem_nodes.data(), int(h.value_size()), w)) {
             h.wave_plan.state = -1;
         } else {
             h.wave_plan.head = upload(w.head, h.stream);
@@ -490,9 +479,7 @@ bool wave_plan_ready(Handle &h)
             h.wave_plan.unused = upload(w.unused, h.stream);
             h.wave_plan.n_unused = int(w.unused.size());
             h.wave_plan.n_chunks = int(w.head.size());
-            // at least what the gradient's staging takes: 3 doubles per unit
-            h.wave_plan.words = std::max(w.max_words, (p1 ? 2 : 1) * 1536 / int(h.value_size()));
-            h.wave_plan.words = (h.wave_plan.words + 3) / 4 * 4;
+            h.wave_plan.words = w.max_words;
             if (!h.brow_ptr.get()) h.brow_ptr = upload(h.pat.brow_ptr, h.stream);
             h.wave_plan.state = 1;
         }

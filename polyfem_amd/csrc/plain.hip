@@ -1805,7 +1805,8 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
 // The factored route's gather.  At gather size 512, the per-contribution
 // gather.  Otherwise the wavefront gather (gather.hip) for meshes of more than
 // wave_units units (node incidences) per CU, and below, or where a node lies in
-// more elements than a wavefront's chunk holds (64 at P2, 128 at P1), the
+// more elements than a wavefront's chunk holds (64 at P2, 128 at P1) or its
+// blocks need more LDS than a workgroup's stages have (wave_limit; P2 FP64), the
 // row-unit gather: 64 units in a workgroup of 128 threads, two for each unit
 // (each forms half of its blocks); where a node has more than 64, 256 units in
 // 256 threads, one each; and where that does not fit either (more than 255

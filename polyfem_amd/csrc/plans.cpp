@@ -191,7 +191,7 @@ WaveShape wave_shape(const std::vector<int32_t> &cnt)
 } // namespace
 
 bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
-                    int value_size, WavePlanHost &out)
+                    int value_size, WavePlanHost &out, int word_limit)
 {
     const std::vector<int32_t> &np = pat.node_ptr, &ni = pat.node_inc, &bp = pat.brow_ptr, &bc = pat.bcol;
     const int NB = n_local, N = pat.n_nodes, cap = 64 * rounds;
@@ -245,7 +245,7 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
             --j;
             for (int32_t b = bp[size_t(j)]; b < bp[size_t(j) + 1]; ++b) --hist[count[size_t(b)]];
         }
-        if (s.n_long > 64) return false;
+        if (s.n_long > 64 || s.words > word_limit) return false;
         WaveHead h{};
         h.row0 = i;
         h.unit0 = np[size_t(i)];
@@ -375,6 +375,16 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
     out.dst = std::move(dst);
     out.desc = std::move(desc);
     out.long_desc = std::move(long_desc);
+    return true;
+}
+
+bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out)
+{
+    const int rounds = wave_rounds(order, n_quad);
+    if (!make_wave_plan(pat, order == 1 ? 4 : 10, elem_nodes, rounds, wave_words(order, value_size), value_size, out,
+                        wave_limit(order, n_quad, value_size)))
+        return false;
+    out.max_words = (std::max(out.max_words, rounds * 1536 / value_size) + 3) / 4 * 4;
     return true;
 }
 

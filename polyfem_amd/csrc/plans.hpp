@@ -86,10 +86,38 @@ struct WavePlanHost {
     int max_words = 0;           // stage words of the largest chunk
 };
 // word_cap: stage words of a chunk of more than one node; value_size: bytes of
-// an entry.  False when a row has more than 64 rounds (at most 2) units,
-// WAVE_BLOCKS blocks or 64 long blocks.
+// an entry; word_limit: stage words of any chunk.  False when a row has more
+// than 64 rounds (at most 2) units, WAVE_BLOCKS blocks or 64 long blocks, or
+// its stage exceeds word_limit or 64 KB.
 bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
-                    int value_size, WavePlanHost &out);
+                    int value_size, WavePlanHost &out, int word_limit = 16384);
+
+// The launch of the wavefront gather, by order, points and bytes of an entry.
+// Units per lane:
+constexpr int wave_rounds(int order, int n_quad) { return order == 1 && n_quad == 1 ? 2 : 1; }
+// Stage words of a chunk of several nodes (three workgroups of four in a CU's
+// LDS for FP32).  Fewer words leave lanes without a unit, more cost
+// wavefronts: P2 mixed 363 us, with 2,496 words 387; P1 mixed 151, with 1,600
+// words 160 and with 2,720 158; P1 FP64 (511,000 tets) 138, with 2,400 142.
+constexpr int wave_words(int order, int value_size) { return order == 2 ? 2528 : value_size == 4 ? 2400 : 1600; }
+// Wavefronts of a workgroup: they share the reference gradients alone.  P2
+// mixed 363 us, with two 376, with one 431 (its waves then are the limit of
+// workgroups per CU); of P2 FP64 one workgroup of eight fills the LDS.
+constexpr int wave_group(int order, int value_size) { return order == 2 && value_size == 8 ? 8 : 4; }
+// Bytes of the reference gradients that a workgroup keeps in LDS, and of its LDS
+constexpr int wave_table(int order, int n_quad, int value_size) { return (order == 1 ? 4 : 10) * n_quad * 4 * value_size; }
+constexpr int WAVE_LDS = 160 * 1024;
+// The most words of a stage: every wavefront of the workgroup has one.  A chunk
+// of one node takes what its blocks need, whatever wave_words says; a node of 52
+// to 64 tets can need more than P2 FP64 has (2,540).
+constexpr int wave_limit(int order, int n_quad, int value_size)
+{
+    return (WAVE_LDS - wave_table(order, n_quad, value_size)) / (wave_group(order, value_size) * value_size) / 4 * 4;
+}
+// The plan the library uses, of stages within wave_limit; max_words: the words
+// of a stage as launched (a multiple of 4, and at least the gradient's staging
+// of 3 doubles per unit).  False where make_wave_plan refuses.
+bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out);
 
 // Chunks of consecutive outputs 0 .. n-1, output i gathering the
 // contributions ptr[i] .. ptr[i+1]-1: a chunk holds at most cap
