@@ -499,7 +499,9 @@ void wave_gather(Handle &h, const void *gloc, double *g, void *values)
                 const int lds = WAVES * p.words * int(sizeof(T));
                 unsigned &grid = GRAD ? p.grid_grad : p.grid;
                 if (grid == 0) {
-                    PF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+                    // the function's limit, not the handle's: one value that every plan fits
+                    PF_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               WAVE_LDS - wave_table(O, Q, int(sizeof(T)))));
                     if (h.n_cu == 0) PF_HIP(hipDeviceGetAttribute(&h.n_cu, hipDeviceAttributeMultiprocessorCount, h.device));
                     int per_cu = 0;
                     PF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * WAVES, size_t(lds)));

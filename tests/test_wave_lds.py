@@ -88,3 +88,27 @@ def test_large_stage_against_oracle(order, tets, precision):
             assert np.abs(u[s:t] - ref[s:t]).max() < TOL[precision] * np.abs(ref[s:t]).max()
         assert np.abs(g[i:j] - gref[i:j]).max() < TOL[precision] * np.abs(gref[i:j]).max()
     assert abs(e - o.energy(x)) < TOL[precision] * abs(o.energy(x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,precision,tets", [(2, "mixed", 64), (1, "fp64", 128)])
+def test_two_live_handles_of_different_stages(order, precision, tets):
+    """The launch limit is the kernel's, which every handle of its order, rule
+    and precision shares: a handle of a smaller stage leaves the others alone."""
+    n = CELLS[order]
+
+    def handle(m):
+        lam, mu = random_lame(m.n_elements, seed=BASE_SEED + 972)
+        x = 0.3 * smooth_displacement(m.nodes, 0.05, 1e-3, BASE_SEED + 973)
+        a = NLAssembler("NeoHookean", m, lame=(lam, mu), precision=precision)
+        return lambda: (*a.assemble_energy_gradient_hessian(x)[1:], a.hessian_values(x))
+
+    box = kuhn_box(n, n, n, order=order)
+    print(f"two handles P{order} {precision}", flush=True)
+    large = handle(union(box, hull_star(tets, order)))
+    first = large()
+    small = handle(box)
+    other = small()
+    for again, want in ((large, first), (small, other), (large, first)):
+        for u, w in zip(again(), want):
+            assert np.array_equal(u, w)
