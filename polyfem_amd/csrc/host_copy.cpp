@@ -7,14 +7,17 @@
 // 1.08 ms with its kernels instead of 1.86, an assembly of 9.5 MB 0.36 instead of
 // 0.63.
 //
-// The pinned memory is a ring of SLOTS slots.  A call leases a ring for its own
-// duration, so handles, threads and streams share no slot; idle rings (at most
-// IDLE_RINGS) wait for the next call and are freed with the last handle.  Arrays
+// The pinned memory is a ring of up to SLOTS pieces, as large as the copy needs.
+// A call leases a ring for its own duration, so handles, threads and streams
+// share no slot; idle rings wait for the next call and are freed with the last
+// handle.  The figures are of a handle in use: up to RING_AFTER its calls take the
+// runtime's copies.  Arrays
 // that DMA reaches by itself (pinned, managed) take the runtime's copy: a
 // Hessian of 9.3 MB into pinned memory takes 234 us with its kernels, through the
 // ring 325.
 #include <algorithm>
 #include <atomic>
+#include <bit>
 #include <cstring>
 #include <exception>
 #include <mutex>
@@ -31,10 +34,19 @@ namespace {
 // but no larger than a slot and no smaller than what the launch of a piece and
 // its event (13 us) cost in transfer time: 24 MB take 439 us in one piece, 514 in
 // pieces of 4 MB, 769 in pieces of 1 MB.
-constexpr int SLOTS = 4, IDLE_RINGS = 4;
+constexpr int SLOTS = 4;
 constexpr size_t SLOT_BYTES = size_t(4) << 20, PIECE_MIN = size_t(1) << 20;
 // below this the copies are latency alone (about 20 us): no ring
 constexpr size_t RING_MIN = size_t(64) << 10;
+// A ring costs 110 to 160 us to allocate and free.  A handle allocates one when
+// its copies, with RESULT_COST for every further result of a call, come to
+// RING_AFTER: about where its gain comes to that.  Handles that are made, called
+// once and dropped do not pay for it (0.7 MB of results: 1,690 us with a ring
+// from the first call on, 1,510 without).
+constexpr size_t RING_AFTER = size_t(16) << 20, RESULT_COST = size_t(512) << 10;
+// Rings of the process, leased and idle (256 MB); calls that find none take the
+// runtime's copies.
+constexpr int MAX_RINGS = 16;
 // Threads that move a slot, the caller's own among them, and the copy from which
 // there are more than one: a thread moves memory that the DMA has just written
 // at about 28 GB/s, half of what the DMA brings, and costs about 20 us to start.
@@ -43,6 +55,7 @@ constexpr size_t MOVERS_MIN = size_t(4) << 20;
 
 struct Ring {
     char *mem = nullptr;
+    size_t bytes = 0;
     hipEvent_t ev[SLOTS] = {};
     int device = -1;
     ~Ring()
@@ -56,15 +69,16 @@ struct Ring {
 std::mutex g_mutex;
 // never destroyed: at the end of the process the runtime may be gone first
 std::vector<std::unique_ptr<Ring>> &g_idle = *new std::vector<std::unique_ptr<Ring>>;
-int g_handles = 0;
+int g_handles = 0, g_rings = 0; // handles alive; rings, leased and idle
 
 // null when pinned memory is not to be had
-std::unique_ptr<Ring> new_ring(int device)
+std::unique_ptr<Ring> new_ring(int device, size_t bytes)
 {
     auto r = std::make_unique<Ring>();
     r->device = device;
+    r->bytes = std::bit_ceil(std::max(bytes, size_t(64) << 10)); // few sizes, so that a ring is seldom replaced
     void *p = nullptr;
-    bool ok = hipHostMalloc(&p, SLOTS * SLOT_BYTES, hipHostMallocDefault) == hipSuccess;
+    bool ok = hipHostMalloc(&p, r->bytes, hipHostMallocDefault) == hipSuccess;
     r->mem = static_cast<char *>(p);
     for (hipEvent_t &e : r->ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (ok) return r;
@@ -72,34 +86,53 @@ std::unique_ptr<Ring> new_ring(int device)
     return nullptr;
 }
 
+// An idle ring of the device with room for bytes; else, if it may be allocated,
+// a new one in the place of a smaller idle one or within MAX_RINGS; else none.
 struct Lease {
     std::unique_ptr<Ring> ring;
     hipStream_t stream;
     bool done = false; // every copy into the ring has ended
-    Lease(int device, hipStream_t s) : stream(s)
+    Lease(int device, hipStream_t s, size_t bytes, bool allocate) : stream(s)
     {
+        std::unique_ptr<Ring> drop;
         {
             std::lock_guard<std::mutex> lock(g_mutex);
-            for (auto &r : g_idle)
-                if (r->device == device) {
-                    ring = std::move(r);
-                    r = std::move(g_idle.back());
-                    g_idle.pop_back();
-                    break;
-                }
+            auto take = [&](bool small) {
+                auto r = std::find_if(g_idle.begin(), g_idle.end(), [&](auto &i) { return i->device == device && (i->bytes < bytes) == small; });
+                if (r == g_idle.end()) return std::unique_ptr<Ring>();
+                std::unique_ptr<Ring> taken = std::move(*r);
+                g_idle.erase(r);
+                return taken;
+            };
+            ring = take(false);
+            if (ring || !allocate) return;
+            drop = take(true);
+            if (!drop && g_rings >= MAX_RINGS) return;
+            g_rings += drop ? 0 : 1;
         }
-        if (!ring) ring = new_ring(device);
+        drop.reset();
+        try {
+            ring = new_ring(device, bytes);
+        } catch (const std::bad_alloc &) {
+        }
+        if (!ring) {
+            std::lock_guard<std::mutex> lock(g_mutex);
+            --g_rings;
+        }
     }
+    Lease(const Lease &) = delete;
     ~Lease()
     {
         if (!ring) return;
         if (!done) (void)hipStreamSynchronize(stream);
         std::unique_ptr<Ring> drop; // freed outside the lock
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_handles > 0 && g_idle.size() < size_t(IDLE_RINGS))
+        if (g_handles > 0) { // g_idle has room for MAX_RINGS
             g_idle.push_back(std::move(ring));
-        else
+        } else {
             drop = std::move(ring);
+            --g_rings;
+        }
     }
 };
 
@@ -124,8 +157,12 @@ void host_copy_handles(int delta)
 {
     std::vector<std::unique_ptr<Ring>> drop;
     std::lock_guard<std::mutex> lock(g_mutex);
+    if (delta > 0) g_idle.reserve(MAX_RINGS); // a lease gives its ring back without allocating
     g_handles += delta;
-    if (g_handles == 0) drop.swap(g_idle);
+    if (g_handles == 0) {
+        g_rings -= int(g_idle.size());
+        drop.swap(g_idle);
+    }
 }
 
 bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
@@ -142,8 +179,13 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
         total += all[i].bytes;
     }
     const int n_items = int(items.size());
+    const size_t piece = std::clamp((total / 4 + 4095) & ~size_t(4095), PIECE_MIN, SLOT_BYTES);
     std::unique_ptr<Lease> lease;
-    if (total >= RING_MIN) lease = std::make_unique<Lease>(h.device, h.stream);
+    if (total >= RING_MIN) {
+        h.copied_to_host += total + size_t(n_items - 1) * RESULT_COST;
+        const size_t pieces = (total + 16 * size_t(n_items)) / piece + 2; // the item that decides has its own
+        lease = std::make_unique<Lease>(h.device, h.stream, std::min(pieces, size_t(SLOTS)) * piece, h.copied_to_host >= RING_AFTER);
+    }
     if (!lease || !lease->ring) {
         for (int i = 0; i < n_all; ++i) {
             PF_HIP(hipMemcpyAsync(all[i].host, all[i].dev, all[i].bytes, hipMemcpyDeviceToHost, h.stream));
@@ -157,7 +199,6 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
         return true;
     }
     Ring &ring = *lease->ring;
-    const size_t piece = std::clamp((total / 4 + 4095) & ~size_t(4095), PIECE_MIN, SLOT_BYTES);
     // pieces of the items, 16-byte aligned in their slots; batch b fills a slot
     // (the item that decides whether the others are written has its own)
     struct Piece {
@@ -183,7 +224,7 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
     const int nb = int(batch.size());
     batch.push_back(pieces.size());
     auto issue = [&](int b) {
-        char *slot = ring.mem + size_t(b % SLOTS) * SLOT_BYTES;
+        char *slot = ring.mem + size_t(b % SLOTS) * piece;
         for (size_t k = batch[size_t(b)]; k < batch[size_t(b) + 1]; ++k)
             PF_HIP(hipMemcpyAsync(slot + pieces[k].at, pieces[k].dev, pieces[k].bytes, hipMemcpyDeviceToHost, h.stream));
         PF_HIP(hipEventRecord(ring.ev[b % SLOTS], h.stream));
@@ -208,7 +249,7 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
     };
     auto move = [&](int b, int t, int n) { // share t of n of batch b
         PF_HIP(hipEventSynchronize(ring.ev[b % SLOTS]));
-        const char *slot = ring.mem + size_t(b % SLOTS) * SLOT_BYTES;
+        const char *slot = ring.mem + size_t(b % SLOTS) * piece;
         const size_t end = pieces[batch[size_t(b) + 1] - 1].at + pieces[batch[size_t(b) + 1] - 1].bytes;
         const size_t lo = end * size_t(t) / size_t(n), hi = end * size_t(t + 1) / size_t(n);
         for (size_t k = batch[size_t(b)]; k < batch[size_t(b) + 1]; ++k) {

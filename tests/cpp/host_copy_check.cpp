@@ -167,6 +167,58 @@ static const std::map<std::string, std::function<void()>> checks = {
             copies(b, {8, 300 * KB, 9 * MB}, 1);
         }
     }},
+    // handles that are made, called a few times and dropped: no ring
+    {"short_lived", [] {
+        for (int k = 0; k < 4; ++k) {
+            Handle h;
+            copies(h, {8, 9 * MB}, 1);
+            Handle g;
+            copies(g, {8, 5000, 300 * KB}, 4);
+        }
+        CHECK(n_alloc == 0);
+    }},
+    // a handle in use: one ring, as large as its copies need, given back with the last handle
+    {"ring_size", [] {
+        {
+            Handle h;
+            copies(h, {8, 20 * KB, 3000 * KB}, 20);
+            CHECK(n_alloc == 1 && largest <= 4 * MB);
+            copies(h, {8, 20 * KB, 300 * KB}, 20);
+            copies(h, {3 * MB}, 20);
+            CHECK(n_alloc == 1);
+            {
+                Handle g; // takes the idle ring at its first call
+                const int waits = n_pageable;
+                copies(g, {8, 20 * KB, 300 * KB}, 1);
+                CHECK(n_pageable == waits);
+            }
+            copies(h, {18 * MB}, 3); // the ring is replaced
+            CHECK(n_alloc == 2 && n_free == 1 && largest <= 16 * MB);
+        }
+        CHECK(n_free == 2 && pinned.empty());
+    }},
+    // more calls at once than idle rings were kept for: no ring is freed between them
+    {"threads", [] {
+        std::atomic<int> at{0};
+        Handle keep;
+        auto work = [&](int n) {
+            return [&, n] {
+                Handle h;
+                for (int k = 0; k < 12; ++k) {
+                    ++at;
+                    for (int spins = 0; at < n * (k + 1) && spins < 1000; ++spins) std::this_thread::yield();
+                    copies(h, {8, 3 * MB}, 1);
+                }
+            };
+        };
+        for (int n : {10, 24}) {
+            std::vector<std::thread> threads;
+            at = 0;
+            for (int t = 0; t < n; ++t) threads.emplace_back(work(n));
+            for (std::thread &t : threads) t.join();
+            CHECK(n_alloc <= std::min(n, 16) && n_free == 0);
+        }
+    }},
     {"errors", [] {
         {
             Handle h;
