@@ -1,20 +1,20 @@
 // Results of the synchronous entry points: device memory into the caller's
 // ordinary host arrays.
 //
-// The runtime copies into pageable memory at about 18 GB/s.  Pieces that go to
-// pinned memory by DMA (56 GB/s) while earlier pieces are moved on to the
-// caller's array end little after the DMA: a projected Hessian of 24 MB takes
-// 1.08 ms with its kernels instead of 1.86, an assembly of 9.5 MB 0.36 instead of
-// 0.63.
+// The runtime copies into pageable memory at about 18 GB/s and waits 15 us for
+// every result.  Pieces that go to pinned memory by DMA (56 GB/s) while earlier
+// pieces are moved on to the caller's array end little after the DMA.  Energy,
+// gradient and Hessian of P1 meshes with their kernels, by the runtime / through
+// the ring, us: 40 KB of results 95 / 60, 2.1 MB 198 / 155, 9.3 MB 635 / 355,
+// 31 MB 1,900 / 855; a projected Hessian of 24 MB 1,860 / 1,050.  These are calls
+// of a handle in use: up to RING_AFTER its calls take the runtime's copies.
 //
 // The pinned memory is a ring of up to SLOTS pieces, as large as the copy needs.
 // A call leases a ring for its own duration, so handles, threads and streams
 // share no slot; idle rings wait for the next call and are freed with the last
-// handle.  The figures are of a handle in use: up to RING_AFTER its calls take the
-// runtime's copies.  Arrays
-// that DMA reaches by itself (pinned, managed) take the runtime's copy: a
-// Hessian of 9.3 MB into pinned memory takes 234 us with its kernels, through the
-// ring 325.
+// handle.  Arrays that DMA reaches by itself (pinned, managed) take the
+// runtime's copy: a Hessian of 9.3 MB into pinned memory takes 234 us with its
+// kernels, through the ring 325.
 #include <algorithm>
 #include <atomic>
 #include <bit>
@@ -36,8 +36,10 @@ namespace {
 // pieces of 4 MB, 769 in pieces of 1 MB.
 constexpr int SLOTS = 4;
 constexpr size_t SLOT_BYTES = size_t(4) << 20, PIECE_MIN = size_t(1) << 20;
-// below this the copies are latency alone (about 20 us): no ring
-constexpr size_t RING_MIN = size_t(64) << 10;
+// One array gains from here on (gradients with their kernels, by the runtime /
+// through the ring, us: 0.7 MB 120 / 120, 1.9 MB 275 / 269, 5.5 MB 745 / 605);
+// several arrays gain at any size, since their copies share one wait.
+constexpr size_t SINGLE_MIN = size_t(2) << 20;
 // A ring costs 110 to 160 us to allocate and free.  A handle allocates one when
 // its copies, with RESULT_COST for every further result of a call, come to
 // RING_AFTER: about where its gain comes to that.  Handles that are made, called
@@ -151,6 +153,17 @@ void copy_plain(Handle &h, const HostCopy &c)
     PF_HIP(hipStreamSynchronize(h.stream));
 }
 
+// the items by the runtime, one after the other: several copies into pageable
+// memory queued at once take longer (95 us for four results of 37 KB, queued 114)
+bool copy_plain(Handle &h, const HostCopy *items, int n_items, const int *stop)
+{
+    for (int i = 0; i < n_items; ++i) {
+        copy_plain(h, items[i]);
+        if (stop && items[i].host == stop && *stop) return false;
+    }
+    return true;
+}
+
 } // namespace
 
 void host_copy_handles(int delta)
@@ -169,7 +182,7 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
 {
     // through the ring, and past it
     std::vector<HostCopy> items, direct;
-    size_t total = 0;
+    size_t total = 0, padded = 0;
     for (int i = 0; i < n_all; ++i) {
         if (dma_reaches(all[i].host)) {
             direct.push_back(all[i]);
@@ -177,28 +190,36 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
         }
         items.push_back(all[i]);
         total += all[i].bytes;
+        padded += (all[i].bytes + 15) & ~size_t(15);
     }
     const int n_items = int(items.size());
     const size_t piece = std::clamp((total / 4 + 4095) & ~size_t(4095), PIECE_MIN, SLOT_BYTES);
     std::unique_ptr<Lease> lease;
-    if (total >= RING_MIN) {
+    if (n_items > 1 || total >= SINGLE_MIN) {
         h.copied_to_host += total + size_t(n_items - 1) * RESULT_COST;
-        const size_t pieces = (total + 16 * size_t(n_items)) / piece + 2; // the item that decides has its own
-        lease = std::make_unique<Lease>(h.device, h.stream, std::min(pieces, size_t(SLOTS)) * piece, h.copied_to_host >= RING_AFTER);
+        const size_t pieces = padded / piece + 2; // the item that decides has its own
+        lease = std::make_unique<Lease>(h.device, h.stream, padded <= piece ? padded : std::min(pieces, size_t(SLOTS)) * piece,
+                                        h.copied_to_host >= RING_AFTER);
     }
-    if (!lease || !lease->ring) {
-        for (int i = 0; i < n_all; ++i) {
-            PF_HIP(hipMemcpyAsync(all[i].host, all[i].dev, all[i].bytes, hipMemcpyDeviceToHost, h.stream));
-            // what *stop guards is not written when it is set
-            if (stop && all[i].host == stop) {
-                PF_HIP(hipStreamSynchronize(h.stream));
-                if (*stop) return false;
-            }
+    if (!lease || !lease->ring) return copy_plain(h, all, n_all, stop);
+    Ring &ring = *lease->ring;
+    // a single piece: nothing to overlap
+    if (padded <= piece) {
+        char *at = ring.mem;
+        for (const HostCopy &c : items) {
+            PF_HIP(hipMemcpyAsync(at, c.dev, c.bytes, hipMemcpyDeviceToHost, h.stream));
+            at += (c.bytes + 15) & ~size_t(15);
         }
         PF_HIP(hipStreamSynchronize(h.stream));
-        return true;
+        lease->done = true;
+        at = ring.mem;
+        for (const HostCopy &c : items) {
+            std::memcpy(c.host, at, c.bytes);
+            if (stop && c.host == stop && *stop) return false;
+            at += (c.bytes + 15) & ~size_t(15);
+        }
+        return copy_plain(h, direct.data(), int(direct.size()), nullptr);
     }
-    Ring &ring = *lease->ring;
     // pieces of the items, 16-byte aligned in their slots; batch b fills a slot
     // (the item that decides whether the others are written has its own)
     struct Piece {
@@ -320,8 +341,7 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
     }
     if (error) std::rethrow_exception(error);
     lease->done = true;
-    for (const HostCopy &c : direct) copy_plain(h, c);
-    return true;
+    return copy_plain(h, direct.data(), int(direct.size()), nullptr);
 }
 
 } // namespace pfgpu

@@ -12,7 +12,8 @@
 
 using namespace pfgpu;
 
-static std::atomic<int> n_alloc{0}, n_free{0}, n_sync{0}, n_pageable{0};
+static std::atomic<int> n_alloc{0}, n_free{0}, n_pageable{0};
+static std::atomic<int> queued{0}, most_queued{0}; // copies into pageable memory since the last wait
 static std::atomic<size_t> largest{0};
 static std::atomic<bool> no_pinned{false}, bad_event{false};
 static std::atomic<const char *> watch{nullptr}; // copies that end at this address are counted
@@ -56,11 +57,14 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
 hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t)
 {
     if (to == watch) ++n_watched;
-    if (!is_pinned(to)) ++n_pageable;
+    if (!is_pinned(to)) {
+        ++n_pageable;
+        if (++queued > most_queued) most_queued = int(queued);
+    }
     std::memcpy(to, from, n);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return ++n_sync, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return queued = 0, hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return *e = reinterpret_cast<hipEvent_t>(std::malloc(1)), hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return std::free(reinterpret_cast<void *>(e)), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
@@ -156,6 +160,24 @@ static const std::map<std::string, std::function<void()>> checks = {
             guarded(h, 0, n);
             guarded(h, 1, n);
         }
+    }},
+    // the runtime copies one result at a time; a handle in use takes several
+    // results of any size through the ring, and a single one from 2 MB on
+    {"small", [] {
+        Handle h;
+        copies(h, {4, 8, 3000, 20 * KB}, 1);
+        CHECK(most_queued == 1 && n_pageable == 4);
+        copies(h, {18 * MB}, 1);
+        CHECK(n_pageable == 4);
+        for (size_t n : {8 * KB, 70 * KB, 300 * KB, 1 * MB}) {
+            n_pageable = 0;
+            copies(h, {4, n}, 1);
+            CHECK(n_pageable == 0);
+            copies(h, {n}, 1);
+            CHECK(n_pageable == 1);
+        }
+        copies(h, {2 * MB}, 1);
+        CHECK(n_pageable == 1);
     }},
     // values that a flag keeps back, with helper threads started and copies in
     // flight, then the same ring under another handle

@@ -11,7 +11,7 @@ from polyfem_amd import PfgpuError, _ffi
 from test_gpu_host_copy import CELLS, case, on_device
 from test_plans import ROOT
 
-CHECKS = ["pinned_destination", "sizes", "kept_back", "short_lived", "ring_size", "threads", "errors"]
+CHECKS = ["pinned_destination", "sizes", "small", "kept_back", "short_lived", "ring_size", "threads", "errors"]
 
 
 @pytest.fixture(scope="module", params=["address,undefined", "thread"])
