@@ -92,6 +92,7 @@ struct GatherPlan {
 // its chunk.
 struct UnitPlan {
     DevBuf chunk_row, udst, bq0, lanes;
+    bool refused = false; // no size of workgroup fits the mesh
     int n_chunks = 0, threads = 0, n_words = 0;
     unsigned grid = 0, grid_grad = 0;
 };

@@ -1834,11 +1834,13 @@ Gather gather_route(Handle &h)
     if (int64_t(h.n_elements) * h.n_local > int64_t(h.n_cu) * wave_units(h.order) && wave_plan_ready(h))
         return Gather::wave;
     ensure_plain_hessian_maps(h);
-    if (9 * int64_t(h.pat.n_blocks) >= (int64_t(1) << 31)) return Gather::contributions;
+    if (h.unit_plan.refused || 9 * int64_t(h.pat.n_blocks) >= (int64_t(1) << 31)) return Gather::contributions;
     if (h.unit_plan.threads || build_unit_plan(h, h.unit_plan, 128, 2)) return Gather::units;
     // dynamic stage + the static tables (row tables, block starts, reference gradients)
     const int64_t lds = int64_t(h.value_size()) * 256 * (h.n_local * 9 + 3) + 8 * 257 + 4 * (256 * h.n_local / 2 + 2) + 1024;
-    return lds <= 160 * 1024 && build_unit_plan(h, h.unit_plan, 256, 1) ? Gather::units : Gather::contributions;
+    if (lds <= 160 * 1024 && build_unit_plan(h, h.unit_plan, 256, 1)) return Gather::units;
+    h.unit_plan.refused = true; // the nodes are not gone through again
+    return Gather::contributions;
 }
 
 // the CSR values (and, with g, the gradient from the local ones in h.loc) from
