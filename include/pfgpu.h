@@ -133,10 +133,13 @@ pfgpu_status pfgpu_set_path(pfgpu_handle *h, int32_t path);
  * configuration of the energy + gradient + Hessian assembly on this handle's
  * mesh at state x (device pointer; 3 timed runs each, after one warm-up) and
  * keeps the fastest.  Candidates: the fused path, the plain path with
- * block-gather workgroups of 128/256/512 threads and Hessian-kernel
- * workgroups of 64/128/256 threads, and the factored path with gather sizes
- * 64/128/256 (its gather chosen by the mesh) and 512 (per contribution).  All candidates give identical results
- * up to the summation order of the path. */
+ * block-gather workgroups of 128/256/512 threads and Hessian-kernel workgroups
+ * of 64/128/256 threads (one size for SaintVenant, FixedCorotational and
+ * MooneyRivlin), and the factored path with its gather chosen by the mesh
+ * (timed at gather sizes 128 and 256) and per contribution (512).  Where the
+ * first one of these wins, gather_threads is the plain path's faster size of 128
+ * and 256.  All candidates give identical results up to the summation order of
+ * the path. */
 typedef struct {
     int32_t path, gather_threads, hessian_threads; /* chosen configuration */
     int32_t candidates;                            /* configurations timed */
@@ -146,8 +149,13 @@ typedef struct {
     double ms_factored;                            /* best factored (negative: not available) */
 } pfgpu_tune_report;
 pfgpu_status pfgpu_autotune(pfgpu_handle *h, const double *x, pfgpu_tune_report *report);
-/* sets a configuration directly (gather_threads in {64,128,256,512},
- * hessian_threads in {64,128,256}) */
+/* Sets a configuration directly (gather_threads in {64,128,256,512},
+ * hessian_threads in {64,128,256}).  On the factored path the gather is chosen by
+ * the mesh at 64, 128 and 256 alike, and per contribution at 512.  On the plain
+ * path, which every path's projected assemblies take, gather_threads is the
+ * workgroup size of the block gather (a node in more elements than that is
+ * PFGPU_ERR_UNSUPPORTED) and hessian_threads that of the Hessian kernel of
+ * NeoHookean and linear elasticity; the other materials' kernel has one size. */
 pfgpu_status pfgpu_set_tuning(pfgpu_handle *h, int32_t path, int32_t gather_threads, int32_t hessian_threads);
 /* replaces ElasticityAssembler::update_lame_params (Assembler.hpp:147-156) */
 pfgpu_status pfgpu_set_lame(pfgpu_handle *h, const double *lambda, const double *mu);

@@ -406,15 +406,19 @@ pfgpu_status pfgpu_autotune(pfgpu_handle *h, const double *x, pfgpu_tune_report 
         r.ms_fused = -1;
         r.ms_factored = -1;
         const int G[3] = {128, 256, 512}, HB[3] = {64, 128, 256};
+        const bool factored = h->material == PFGPU_NEOHOOKEAN || h->material == PFGPU_LINEAR_ELASTICITY;
+        double plain_ms[3] = {1e300, 1e300, 1e300}; // by gather size
         try {
             for (int gi = 0; gi < 3; ++gi)
-                for (int hi = 0; hi < 3; ++hi) {
+                // the other materials' Hessian kernel has one size (points.hip)
+                for (int hi = factored ? 0 : 2; hi < 3; ++hi) {
                     h->path = PFGPU_PATH_PLAIN;
                     h->tune_gather_threads = G[gi];
                     h->tune_hessian_threads = HB[hi];
                     const double ms = time_config();
                     r.candidates++;
                     if (G[gi] == 256 && HB[hi] == 256) r.ms_plain_default = ms;
+                    plain_ms[gi] = std::min(plain_ms[gi], ms);
                     if (ms < r.ms) {
                         r.ms = ms;
                         r.path = PFGPU_PATH_PLAIN;
@@ -422,27 +426,29 @@ pfgpu_status pfgpu_autotune(pfgpu_handle *h, const double *x, pfgpu_tune_report 
                         r.hessian_threads = HB[hi];
                     }
                 }
-            // the factored path keeps the plain winner's Hessian-kernel size
-            // (used by its PSD-projected assemblies)
+            // The factored path keeps the plain winner's Hessian-kernel size (used
+            // by its PSD-projected assemblies).  Up to 256 its own gather depends
+            // on the mesh alone, so that the times of 128 and 256 are two of the
+            // same kernels: the size kept is the better one of the plain gather,
+            // which the projected assemblies take too.
             h->tune_hessian_threads = r.hessian_threads;
-            const int GF[4] = {64, 128, 256, 512};
-            if (h->material == PFGPU_NEOHOOKEAN || h->material == PFGPU_LINEAR_ELASTICITY)
-                for (int gi = 0; gi < 4; ++gi) {
-                    h->path = PFGPU_PATH_FACTORED;
-                    h->tune_gather_threads = GF[gi];
-                    try {
-                        const double ms = time_config();
-                        r.candidates++;
-                        if (r.ms_factored < 0 || ms < r.ms_factored) r.ms_factored = ms;
-                        if (ms < r.ms) {
-                            r.ms = ms;
-                            r.path = PFGPU_PATH_FACTORED;
-                            r.gather_threads = GF[gi];
-                        }
-                    } catch (const Error &e) {
-                        if (e.status != PFGPU_ERR_UNSUPPORTED) throw;
+            const int by_mesh = plain_ms[0] <= plain_ms[1] ? G[0] : G[1];
+            for (int gi = 0; factored && gi < 3; ++gi) {
+                h->path = PFGPU_PATH_FACTORED;
+                h->tune_gather_threads = G[gi];
+                try {
+                    const double ms = time_config();
+                    r.candidates++;
+                    if (r.ms_factored < 0 || ms < r.ms_factored) r.ms_factored = ms;
+                    if (ms < r.ms) {
+                        r.ms = ms;
+                        r.path = PFGPU_PATH_FACTORED;
+                        r.gather_threads = G[gi] > 256 ? G[gi] : by_mesh;
                     }
+                } catch (const Error &e) {
+                    if (e.status != PFGPU_ERR_UNSUPPORTED) throw;
                 }
+            }
             h->path = PFGPU_PATH_FUSED;
             try {
                 r.ms_fused = time_config();
@@ -464,9 +470,9 @@ pfgpu_status pfgpu_autotune(pfgpu_handle *h, const double *x, pfgpu_tune_report 
         h->path = r.path;
         h->tune_gather_threads = r.gather_threads ? r.gather_threads : 256;
         h->tune_hessian_threads = r.hessian_threads ? r.hessian_threads : 256;
-        // one call in the chosen configuration builds its tables (gather
-        // plans are built for one workgroup size), so that the caller's
-        // first assembly does not
+        // one call in the chosen configuration builds its tables (the plain and
+        // per-contribution gathers keep the plan of one workgroup size), so that
+        // the caller's first assembly does not
         egh_dev(*h, x, de, dg, dv);
         PF_HIP(hipStreamSynchronize(h->stream));
         *report = r;
