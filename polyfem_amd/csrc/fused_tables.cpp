@@ -15,9 +15,9 @@
 #include <algorithm>
 #include <array>
 #include <numeric>
-#include <thread>
 
 #include "fused.hpp"
+#include "parallel.hpp"
 
 namespace pfgpu {
 
@@ -273,15 +273,9 @@ FusedTables build_fused_tables(const Pattern &pat, int n_local, const int32_t *e
             }
         }
     };
-    {
-        const int T = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-        std::vector<std::thread> th;
-        for (int w = 0; w < T; ++w)
-            th.emplace_back([&, w] {
-                for (int p = w; p < P; p += T) build_one(p);
-            });
-        for (auto &x : th) x.join();
-    }
+    parallel_parts([&](int w, int n) {
+        for (int p = w; p < P; p += n) build_one(p);
+    });
 
     // concatenate
     t.desc.assign(size_t(P) * PD_STRIDE, 0);

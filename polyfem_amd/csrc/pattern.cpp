@@ -8,9 +8,9 @@
 // node adjacency (nodes sharing an element) times a full 3x3 block, which is
 // what this file builds directly, without triplets.
 #include <algorithm>
-#include <thread>
 
 #include "common.hpp"
+#include "parallel.hpp"
 
 namespace pfgpu {
 
@@ -18,17 +18,10 @@ namespace {
 
 template <typename F> void parallel_for(int n, F &&f)
 {
-    const int T = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    if (n < 4096 || T == 1) {
+    if (n < 4096)
         f(0, n);
-        return;
-    }
-    std::vector<std::thread> th;
-    for (int t = 0; t < T; ++t) {
-        const int s = int(int64_t(t) * n / T), e = int(int64_t(t + 1) * n / T);
-        th.emplace_back([&f, s, e] { f(s, e); });
-    }
-    for (auto &t : th) t.join();
+    else
+        parallel_ranges(n, f);
 }
 
 void incidence(int n_elements, int n_local, const int32_t *conn, int n_items, std::vector<int32_t> &ptr,

@@ -3,9 +3,9 @@
 // only, so that tests can build and check the plans on the CPU.
 #include <algorithm>
 #include <atomic>
-#include <thread>
 #include <utility>
 
+#include "parallel.hpp"
 #include "plans.hpp"
 
 namespace pfgpu {
@@ -145,10 +145,7 @@ bool make_unit_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
             chunk_lanes(pieces, nb, i1 - i0, n_lanes, lanes.data() + size_t(ci) * size_t(n_lanes + 1));
         }
     };
-    const int nt = int(std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nt; ++t) pool.emplace_back(fill, int(int64_t(nc) * t / nt), int(int64_t(nc) * (t + 1) / nt));
-    for (std::thread &th : pool) th.join();
+    parallel_ranges(nc, fill);
     if (!fits) return false;
     out.chunk_row = std::move(c);
     out.udst = std::move(dst);
@@ -199,13 +196,7 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
     std::vector<uint8_t> count(size_t(pat.n_blocks));
     std::vector<uint16_t> upos(size_t(np[size_t(N)]) * NB);
     std::atomic<bool> fits{true};
-    const int nt = int(std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
-    auto parallel = [&](int n, auto &&f) {
-        std::vector<std::thread> pool;
-        for (int t = 0; t < nt; ++t) pool.emplace_back(f, int(int64_t(n) * t / nt), int(int64_t(n) * (t + 1) / nt));
-        for (std::thread &th : pool) th.join();
-    };
-    parallel(N, [&](int i0, int i1) {
+    parallel_ranges(N, [&](int i0, int i1) {
         for (int i = i0; i < i1; ++i) {
             const int32_t r0 = bp[size_t(i)], deg = bp[size_t(i) + 1] - r0;
             if (np[size_t(i) + 1] - np[size_t(i)] > cap || deg > WAVE_BLOCKS) {
@@ -274,7 +265,7 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
     const int nc = int(head.size());
     std::vector<uint32_t> desc(static_cast<size_t>(nw), 0), long_desc(size_t(2 * nl));
     std::vector<uint16_t> dst(size_t(nc) * size_t(cap) * size_t(NB), 0);
-    parallel(nc, [&](int c0, int c1) {
+    parallel_ranges(nc, [&](int c0, int c1) {
         // per output block: its contributions (unit, b), in unit order
         std::vector<int32_t> ptr, list, order, next, sorted, row_of, pos(size_t(cap) * size_t(NB));
         for (int ci = c0; ci < c1; ++ci) {
@@ -462,10 +453,7 @@ bool make_contrib_plan(const Pattern &pat, const std::vector<int32_t> &ptr, cons
             }
         }
     };
-    const int nt = int(std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nt; ++t) pool.emplace_back(fill, int(int64_t(nc) * t / nt), int(int64_t(nc) * (t + 1) / nt));
-    for (std::thread &th : pool) th.join();
+    parallel_ranges(nc, fill);
     out.chunk = std::move(c);
     out.slot = std::move(slot);
     out.meta = std::move(meta);
