@@ -189,9 +189,9 @@ void solver_release(Handle &h);
 
 // ---- misc kernels (reduce.hip) ----------------------------------------
 void build_device_pattern(Handle &h);
-// returns true when every value in the device array is finite
-// *flag (device) becomes 1 where v has a non-finite entry, else 0
+// a device flag: 1 where the device array has a non-finite entry, else 0
 int *count_nonfinite(Handle &h, const void *dev, int64_t n, bool is_float);
+// returns true when every value in the device array is finite
 bool all_finite(Handle &h, const void *dev, int64_t n, bool is_float);
 // device results into host arrays (host_copy.cpp), complete on return; with stop,
 // one of the items' hosts, false as soon as it arrives non-zero (later items are

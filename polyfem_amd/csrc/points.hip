@@ -38,7 +38,7 @@ template <typename T> __device__ __forceinline__ void map3(const T *A, const T *
 #pragma unroll
     for (int i = 0; i < 3; ++i) out[i] = A[3 * i] * r[0] + A[3 * i + 1] * r[1] + A[3 * i + 2] * r[2];
 }
-// out = s A r for symmetric A (00 11 22 01 02 12)
+// out = A r for symmetric A (00 11 22 01 02 12)
 template <typename T> __device__ __forceinline__ void map_sym(const T *A, const T *r, T *out)
 {
     out[0] = A[0] * r[0] + A[3] * r[1] + A[4] * r[2];

@@ -46,7 +46,7 @@ constexpr int SPMV_LANES = PF_SPMV_LANES; // lanes per block row of the block-sp
 // at the tolerance (r.r <= S_TOL); S_ITER counts the updates taken
 // S_OLD, S_STOP: r.z and the flag of the running iteration as the update kernel
 // leaves them for the direction kernel, which writes S_RZ and S_FLAG
-enum { S_RR, S_PQ, S_ALPHA, S_BETA, S_RZ, S_FLAG, S_B2, S_GD, S_E0, S_E1, S_M, S_F, S_TOL, S_ITER, S_OLD, S_STOP, S_COUNT };
+enum { S_RR, S_ALPHA, S_RZ, S_FLAG, S_B2, S_GD, S_E0, S_E1, S_M, S_F, S_TOL, S_ITER, S_OLD, S_STOP, S_COUNT };
 enum { CG_RUNNING = 0, CG_CURVATURE = 1, CG_TOLERANCE = 2 };
 
 // the sum over the workgroup, in every thread: the tree s[t] += s[t + w],
@@ -166,7 +166,6 @@ __global__ __launch_bounds__(BLOCK) void k_pcg_update(int n_nodes, int n_pq, dou
     const double v = sum_partials(part_pq, n_pq, sh), old = scal[S_RZ], flag = scal[S_FLAG];
     const double a = v > 0.0 && old > 0.0 && flag == 0.0 ? old / v : 0.0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        scal[S_PQ] = v;
         scal[S_ALPHA] = a;
         scal[S_OLD] = old;
         scal[S_STOP] = !(v > 0.0) && old > 0.0 && flag == 0.0 ? double(CG_CURVATURE) : flag;
@@ -232,7 +231,6 @@ __global__ __launch_bounds__(BLOCK) void k_cg_direction(int n_nodes, double *__r
     if (blockIdx.x == 0) { // uniform over the workgroup
         const double rr = sum_partials(part_rr, int(gridDim.x), s);
         if (threadIdx.x == 0) {
-            scal[S_BETA] = beta;
             if (stop == 0.0) {
                 scal[S_RZ] = rz;
                 scal[S_RR] = rr;
