@@ -37,7 +37,8 @@
 // two threads per unit, a lane per piece of a block):
 // 384,000 P2 tets NeoHookean mixed 450 -> 363 us, 44,600 P2 tets linear
 // elasticity FP64 117 -> 87, 912,000 P1 tets mixed 162 -> 151, 511,000 P1 tets
-// FP64 138 (see gather_route in plain.hip for smaller meshes).
+// FP64 138 (lattice meshes; see gather_route in plain.hip for smaller ones and
+// wave_share in plans.hpp for P1 meshes that do not take it).
 #include "dispatch.hpp"
 #include "factors.hpp"
 #include "plans.hpp"
@@ -459,14 +460,16 @@ __global__ __launch_bounds__(BLOCK) void k_zero_nodes(int n, const int32_t *__re
 } // namespace
 
 // the wavefront plan of the handle; false when a node has too many incident
-// elements for one chunk, or blocks for a stage that the workgroup's LDS holds
-// (the row-unit gather then serves the handle)
+// elements for one chunk, or blocks for a stage that the workgroup's LDS holds,
+// or the chunks would have too few units (wave_share; the row-unit gather then
+// serves the handle)
 bool wave_plan_ready(Handle &h)
 {
     if (h.wave_plan.state == 0) {
         WavePlanHost w;
-        if (9 * h.pat.n_blocks >= (int64_t(1) << 31) ||
-            !plan_wave_gather(h.pat, h.order, h.n_quad, h.h_elem_nodes.data(), int(h.value_size()), w)) {
+        const double least = least_wave_share(h.pat, h.order, h.n_quad, int(h.value_size()));
+        if (9 * h.pat.n_blocks >= (int64_t(1) << 31) || least > 1 ||
+            !plan_wave_gather(h.pat, h.order, h.n_quad, h.h_elem_nodes.data(), int(h.value_size()), w, least)) {
             h.wave_plan.state = -1;
         } else {
             h.wave_plan.head = upload(w.head, h.stream);
@@ -492,7 +495,7 @@ void wave_gather(Handle &h, const void *gloc, double *g, void *values)
 {
     WavePlan &p = h.wave_plan;
     dispatch<true>(h, [&]<typename T, int O, int Q, int M>() {
-        if constexpr (M == MAT_NH || M == MAT_LE) {
+        if constexpr ((M == MAT_NH || M == MAT_LE) && wave_share(O, Q, sizeof(T), false) <= 1) {
             auto go = [&]<bool GRAD>() {
                 constexpr int WAVES = wave_group(O, sizeof(T));
                 auto kern = k_gather_wave<T, O, Q, GRAD>;
@@ -521,6 +524,8 @@ void wave_gather(Handle &h, const void *gloc, double *g, void *values)
             } else {
                 go.template operator()<false>();
             }
+        } else {
+            fail(PFGPU_ERR_INVALID_STATE, "the wavefront gather does not cover this rule or material");
         }
     });
     PF_LAUNCH_CHECK();

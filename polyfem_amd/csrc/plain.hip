@@ -1804,14 +1804,15 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
 
 // The factored route's gather.  At gather size 512, the per-contribution
 // gather.  Otherwise the wavefront gather (gather.hip) for meshes of more than
-// wave_units units (node incidences) per CU, and below, or where a node lies in
-// more elements than a wavefront's chunk holds (64 at P2, 128 at P1) or its
-// blocks need more LDS than a workgroup's stages have (wave_limit; P2 FP64), the
-// row-unit gather: 64 units in a workgroup of 128 threads, two for each unit
-// (each forms half of its blocks); where a node has more than 64, 256 units in
-// 256 threads, one each; and where that does not fit either (more than 255
-// elements, or P2 FP64, whose staged blocks exceed the 160 KB of LDS), the
-// per-contribution gather.
+// wave_units units (node incidences) per CU whose rows fill its chunks
+// (wave_share), and below, or where a node lies in more elements than a
+// wavefront's chunk holds (64 at P2, 128 at P1) or its blocks need more LDS than a
+// workgroup's stages have (wave_limit; P2 FP64), the row-unit gather: 64 units in
+// a workgroup of 128 threads, two for each unit (each forms half of its blocks);
+// where a node has more than 64, and on large P1 meshes in FP32, 256 units in 256
+// threads, one each; and where that does not fit either (more than 255 elements,
+// or P2 FP64, whose staged blocks exceed the 160 KB of LDS), the per-contribution
+// gather.
 //
 // A chunk of the wavefront gather is one wavefront's work from end to end: on
 // small meshes two threads per unit finish sooner, and up to a few chunks per
@@ -1822,7 +1823,9 @@ template <typename T, int O, int Q> void launch_unit_gather(Handle &h, UnitPlan 
 // 195 / 163 at 56^3; P2 FP64 20.5 / 31.5 at 4^3, 70.6 / 72.0 at 16^3, 93.5 /
 // 74.1 at 18^3; P2 mixed 23.1 / 27.3 at 10^3, 42.3 / 43.3 at 16^3, 52.9 / 48.4
 // at 18^3, 450 / 363 at 40^3.  256 units of one thread each took 14.4 us where
-// 64 of two take 12.3 (P1 FP64, 4^3), 24.3 / 19.2 (P2 mixed, 4^3).
+// 64 of two take 12.3 (P1 FP64, 4^3), 24.3 / 19.2 (P2 mixed, 4^3), 325 / 269
+// (769,000 unstructured P1 tets FP64), but 22.4 / 20.9 at 48,000 P1 tets in FP32,
+// 40.6 / 40.5 at 162,000 (the Hessian alone 32.7 / 35.1) and 135 / 150 at 769,000.
 constexpr int wave_units(int order) { return order == 2 ? 1024 : 2048; }
 enum class Gather { wave, units, contributions };
 Gather gather_route(Handle &h)
@@ -1831,11 +1834,12 @@ Gather gather_route(Handle &h)
         fail(PFGPU_ERR_UNSUPPORTED, "the factored Hessian covers NeoHookean and linear elasticity");
     if (h.tune_gather_threads > 256) return Gather::contributions;
     if (h.n_cu == 0) PF_HIP(hipDeviceGetAttribute(&h.n_cu, hipDeviceAttributeMultiprocessorCount, h.device));
-    if (int64_t(h.n_elements) * h.n_local > int64_t(h.n_cu) * wave_units(h.order) && wave_plan_ready(h))
-        return Gather::wave;
+    const bool large = int64_t(h.n_elements) * h.n_local > int64_t(h.n_cu) * wave_units(h.order);
+    if (large && wave_plan_ready(h)) return Gather::wave;
     ensure_plain_hessian_maps(h);
     if (h.unit_plan.refused || 9 * int64_t(h.pat.n_blocks) >= (int64_t(1) << 31)) return Gather::contributions;
-    if (h.unit_plan.threads || build_unit_plan(h, h.unit_plan, 128, 2)) return Gather::units;
+    const bool wide = large && h.order == 1 && h.precision == PFGPU_MIXED;
+    if (h.unit_plan.threads || (!wide && build_unit_plan(h, h.unit_plan, 128, 2))) return Gather::units;
     // dynamic stage + the static tables (row tables, block starts, reference gradients)
     const int64_t lds = int64_t(h.value_size()) * 256 * (h.n_local * 9 + 3) + 8 * 257 + 4 * (256 * h.n_local / 2 + 2) + 1024;
     if (lds <= 160 * 1024 && build_unit_plan(h, h.unit_plan, 256, 1)) return Gather::units;

@@ -188,7 +188,7 @@ WaveShape wave_shape(const std::vector<int32_t> &cnt)
 } // namespace
 
 bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
-                    int value_size, WavePlanHost &out, int word_limit)
+                    int value_size, WavePlanHost &out, int word_limit, double least_share)
 {
     const std::vector<int32_t> &np = pat.node_ptr, &ni = pat.node_inc, &bp = pat.brow_ptr, &bc = pat.bcol;
     const int NB = n_local, N = pat.n_nodes, cap = 64 * rounds;
@@ -263,6 +263,8 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
         i = j;
     }
     const int nc = int(head.size());
+    out.share = nc ? double(np[size_t(N)]) / (double(nc) * cap) : 1.0;
+    if (out.share < least_share) return false;
     std::vector<uint32_t> desc(static_cast<size_t>(nw), 0), long_desc(size_t(2 * nl));
     std::vector<uint16_t> dst(size_t(nc) * size_t(cap) * size_t(NB), 0);
     parallel_ranges(nc, [&](int c0, int c1) {
@@ -369,14 +371,22 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
     return true;
 }
 
-bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out)
+bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out,
+                      double least_share)
 {
     const int rounds = wave_rounds(order, n_quad);
     if (!make_wave_plan(pat, order == 1 ? 4 : 10, elem_nodes, rounds, wave_words(order, value_size), value_size, out,
-                        wave_limit(order, n_quad, value_size)))
+                        wave_limit(order, n_quad, value_size), least_share))
         return false;
     out.max_words = (std::max(out.max_words, rounds * 1536 / value_size) + 3) / 4 * 4;
     return true;
+}
+
+double least_wave_share(const Pattern &pat, int order, int n_quad, int value_size)
+{
+    bool large = false;
+    for (int i = 0; i < pat.n_nodes; ++i) large |= pat.node_ptr[size_t(i) + 1] - pat.node_ptr[size_t(i)] > 64;
+    return wave_share(order, n_quad, value_size, large);
 }
 
 bool segment_chunks(const int32_t *ptr, int64_t n, int cap, std::vector<int32_t> &c)

@@ -84,13 +84,15 @@ struct WavePlanHost {
     std::vector<uint32_t> desc, long_desc;
     std::vector<int32_t> unused; // nodes outside the chunks: no element uses them
     int max_words = 0;           // stage words of the largest chunk
+    double share = 0;            // of the chunks' lanes and rounds with a unit
 };
 // word_cap: stage words of a chunk of more than one node; value_size: bytes of
 // an entry; word_limit: stage words of any chunk.  False when a row has more
-// than 64 rounds (at most 2) units, WAVE_BLOCKS blocks or 64 long blocks, or
-// its stage exceeds word_limit or 64 KB.
+// than 64 rounds (at most 2) units, WAVE_BLOCKS blocks or 64 long blocks, its
+// stage exceeds word_limit or 64 KB, or the share is below least_share (found
+// before the lanes are dealt).
 bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
-                    int value_size, WavePlanHost &out, int word_limit = 16384);
+                    int value_size, WavePlanHost &out, int word_limit = 16384, double least_share = 0);
 
 // The launch of the wavefront gather, by order, points and bytes of an entry.
 // Units per lane:
@@ -117,7 +119,34 @@ constexpr int wave_limit(int order, int n_quad, int value_size)
 // The plan the library uses, of stages within wave_limit; max_words: the words
 // of a stage as launched (a multiple of 4, and at least the gradient's staging
 // of 3 doubles per unit).  False where make_wave_plan refuses.
-bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out);
+bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *elem_nodes, int value_size, WavePlanHost &out,
+                      double least_share = 0);
+// The share from which the wavefront gather is the faster one on a large mesh
+// (above 1: never), which wave_plan_ready passes as least_share; large_node: a
+// node lies in more than 64 elements, so that the row-unit gather takes 256 units
+// in a workgroup instead of 64.
+//
+// A chunk costs nearly the same whatever its lanes hold, and P1 rows of an
+// unstructured mesh, with blocks of all counts, fill a stage with few units.
+// E + G + H of 0.6 to 1.1 million P1 tets, wavefronts / the better row units, us:
+//   one point FP64: lattice (share 0.73) 175 / 200, BCC points moved by 5 %
+//   (0.68) 255 / 255, by 15 % (0.53) 292 / 259, by 25 % (0.30) 447 / 269, random
+//   points (0.23) 586 / 291; with large nodes 267 / 307 (0.65), 303 / 315 (0.53),
+//   460 / 331 (0.30), 604 / 381 (0.23)
+//   one point FP32: lattice (0.93) 93 / 102, BCC 5 % (0.91) 129 / 128, 15 %
+//   (0.84) 130 / 131 and with another numbering 144 / 136, 25 % (0.79) 143 / 135;
+//   with large nodes 134 / 132 (0.91), 142 / 128 (0.84), 163 / 151 (0.81)
+//   four points, FP64 and FP32: lattice 381 / 355 and 178 / 156, BCC 5 % 500 / 452
+//   and 225 / 202
+// At P2 the wavefronts are the faster ones throughout (161,000 tets of BCC points
+// moved by 25 %: FP64 285 / 389, FP32 179 / 196).
+constexpr double wave_share(int order, int n_quad, int value_size, bool large_node)
+{
+    if (order == 2) return 0;
+    if (n_quad != 1) return 2;
+    return value_size == 8 ? (large_node ? 0.55 : 0.7) : large_node ? 2 : 0.88;
+}
+double least_wave_share(const Pattern &pat, int order, int n_quad, int value_size);
 
 // Chunks of consecutive outputs 0 .. n-1, output i gathering the
 // contributions ptr[i] .. ptr[i+1]-1: a chunk holds at most cap
