@@ -242,9 +242,22 @@ template <typename T> struct PointForm<T, MAT_MR> {
 // the row and reduction work per element is shared by fewer lanes (P2 Hessian
 // with its gather, mixed: 384,000 tets 802 us against 840 us with four lanes
 // and 808 us with one; 10,368 tets 46 us against 43 us and 69 us).
-template <typename T, int MAT> constexpr int points_lanes(int nq)
+//
+// On large P1 meshes (from 16,384 elements) two lanes are the better ones for
+// six points, of which four lanes leave a quarter idle, and for SaintVenant's four
+// points in FP64 too: with ten blocks per element the points' forms are most of the
+// work, and there are elements enough.  843,648 P1 tets, Hessian with its gather,
+// two / four lanes, us: SaintVenant six points FP64 536 / 551, FP32 278 / 310,
+// four points FP64 435 / 450 (one thread per element with the form of this material
+// alone: 502, 267 and 402); FixedCorotational 995 / 1,274 and 588 / 686,
+// MooneyRivlin 766 / 941 and 354 / 444; 24,576 tets: SaintVenant 27.1 / 30.1, 19.6 /
+// 19.4 and 25.3 / 26.3; 1,296 tets 14.8 / 13.3, 13.2 / 11.9 and 13.4 / 12.1.
+constexpr int POINTS_LARGE = 16384;
+template <typename T, int MAT> constexpr int points_lanes(int order, int nq, bool large)
 {
-    return nq == 1 ? 1 : MAT == MAT_SV && sizeof(T) == 4 && nq == 4 ? 2 : 4;
+    if (nq == 1) return 1;
+    if (MAT == MAT_SV && sizeof(T) == 4 && nq == 4) return 2;
+    return order == 1 && large && (nq == 6 || (MAT == MAT_SV && nq == 4)) ? 2 : 4;
 }
 
 // hloc as k_hessian writes it: block s of element e at
@@ -255,11 +268,11 @@ template <typename T, int MAT> constexpr int points_lanes(int nq)
 // the pairs' 9 values are staged in LDS, and the lanes that store the run add
 // the two pairs of an element (finishing the sum by quad permutes instead
 // costs 20 more VALU instructions per block, 25 % of the kernel's).
-template <typename T, int ORDER, int NQ, int MAT>
+template <typename T, int ORDER, int NQ, int MAT, int LPE>
 __global__ __launch_bounds__(BLOCK) void k_hessian_points(DevMesh<T> m, const double *__restrict__ x, T *__restrict__ hloc)
 {
     constexpr int NB = NLocal<ORDER>::value, NBLK = NB * (NB + 1) / 2;
-    constexpr int LPE = points_lanes<T, MAT>(NQ), QPL = (NQ + LPE - 1) / LPE, EPW = 64 / LPE, RUN = EPW * 9;
+    constexpr int QPL = (NQ + LPE - 1) / LPE, EPW = 64 / LPE, RUN = EPW * 9;
     constexpr int HALVES = LPE == 4 ? 2 : 1, NOUT = (RUN + 63) / 64;
     __shared__ __align__(16) T stage[BLOCK / 64][RUN * HALVES];
     // reference gradients (r0 r1 r2) and weight per (point, node)
@@ -359,11 +372,18 @@ __global__ __launch_bounds__(BLOCK) void k_hessian_points(DevMesh<T> m, const do
 void points_hessian(Handle &h, const double *x, void *hloc)
 {
     dispatch(h, [&]<typename T, int O, int Q, int M>() {
-        if constexpr (M == MAT_SV || M == MAT_FC || M == MAT_MR)
-            k_hessian_points<T, O, Q, M><<<grid_for(int64_t(h.n_elements) * points_lanes<T, M>(Q)), BLOCK, 0, h.stream>>>(
-                h.mesh<T>(), x, static_cast<T *>(hloc));
-        else
+        if constexpr (M == MAT_SV || M == MAT_FC || M == MAT_MR) {
+            auto go = [&]<int LPE>() {
+                k_hessian_points<T, O, Q, M, LPE><<<grid_for(int64_t(h.n_elements) * LPE), BLOCK, 0, h.stream>>>(h.mesh<T>(), x,
+                                                                                                             static_cast<T *>(hloc));
+            };
+            if (h.n_elements < POINTS_LARGE)
+                go.template operator()<points_lanes<T, M>(O, Q, false)>();
+            else
+                go.template operator()<points_lanes<T, M>(O, Q, true)>();
+        } else {
             fail(PFGPU_ERR_INVALID_STATE, "the point-parallel Hessian covers SaintVenant, FixedCorotational and MooneyRivlin");
+        }
     });
     PF_LAUNCH_CHECK();
 }
