@@ -29,9 +29,9 @@
 // 356 us for the 384,000-tet mesh below.)
 //
 // What bounds it: instruction issue and LDS latency of few wavefronts.  Of
-// 340 us for 384,000 P2 tets mixed, leaving out the sums takes 90 us off, the
-// stores 72 and the gradient 20; formation alone needs 137 and its memory
-// traffic about 150.  More wavefronts (16 instead of 12 per CU, by smaller
+// 340 us under the profiler (300 in a timed pass) for 384,000 P2 tets mixed,
+// leaving out the sums takes 90 us off, the stores 72 and the gradient 20;
+// formation alone needs 137 and its memory traffic about 150.  More wavefronts (16 instead of 12 per CU, by smaller
 // chunks) gave nothing, since the smaller chunks leave lanes idle.
 // E + G + H with this gather against the row-unit gather (64 units per workgroup,
 // two threads per unit, a lane per piece of a block):
