@@ -12,7 +12,7 @@ struct pfgpu_handle {
     int n_elements = 0, n_nodes = 0, n_vertices = 0, n_dofs = 0;
     hipStream_t stream = nullptr;
     int device = 0;
-    size_t copied_to_host = 0; // of results, until a ring pays (host_copy.cpp)
+    size_t copied_to_host = 0, host_ring = 0; // results copied so far and the ring for the largest (host_copy.cpp)
 
     pfgpu::Pattern pat;
     std::vector<int32_t> h_elem_nodes; // host copy, element-major (E x n_local)

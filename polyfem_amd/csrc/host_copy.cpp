@@ -7,7 +7,7 @@
 // gradient and Hessian of P1 meshes with their kernels, by the runtime / through
 // the ring, us: 40 KB of results 95 / 60, 2.1 MB 198 / 155, 9.3 MB 635 / 355,
 // 31 MB 1,900 / 855; a projected Hessian of 24 MB 1,860 / 1,050.  These are calls
-// of a handle in use: up to RING_AFTER its calls take the runtime's copies.
+// of a handle in use: its first ones take the runtime's copies (RING_PAYS).
 //
 // The pinned memory is a ring of up to SLOTS pieces, as large as the copy needs.
 // A call leases a ring for its own duration, so handles, threads and streams
@@ -40,12 +40,14 @@ constexpr size_t SLOT_BYTES = size_t(4) << 20, PIECE_MIN = size_t(1) << 20;
 // through the ring, us: 0.7 MB 120 / 120, 1.9 MB 275 / 269, 5.5 MB 745 / 605);
 // several arrays gain at any size, since their copies share one wait.
 constexpr size_t SINGLE_MIN = size_t(2) << 20;
-// A ring costs 110 to 160 us to allocate and free.  A handle allocates one when
-// its copies, with RESULT_COST for every further result of a call, come to
-// RING_AFTER: about where its gain comes to that.  Handles that are made, called
-// once and dropped do not pay for it (0.7 MB of results: 1,690 us with a ring
-// from the first call on, 1,510 without).
-constexpr size_t RING_AFTER = size_t(16) << 20, RESULT_COST = size_t(512) << 10;
+// A ring costs 0.1 to 0.2 ms per MB to allocate and first use (less where the
+// process has freed pinned memory before), and gains 0.03 ms per MB copied.  A
+// handle allocates one, for its largest copy so far, when its earlier copies (with
+// RESULT_COST for every further result of a call) or the one at hand come to
+// RING_PAYS times that.  Handles that are made, called once and dropped do not
+// pay for it (0.7 MB of results: 1,690 us with a ring from the first call on, 1,510
+// without; the first derivatives of a process, 25 MB: 3.8 ms and 2.3).
+constexpr size_t RING_PAYS = 4, RESULT_COST = size_t(512) << 10;
 // Rings of the process, leased and idle (256 MB); calls that find none take the
 // runtime's copies.
 constexpr int MAX_RINGS = 16;
@@ -78,7 +80,7 @@ std::unique_ptr<Ring> new_ring(int device, size_t bytes)
 {
     auto r = std::make_unique<Ring>();
     r->device = device;
-    r->bytes = std::bit_ceil(std::max(bytes, size_t(64) << 10)); // few sizes, so that a ring is seldom replaced
+    r->bytes = bytes;
     void *p = nullptr;
     bool ok = hipHostMalloc(&p, r->bytes, hipHostMallocDefault) == hipSuccess;
     r->mem = static_cast<char *>(p);
@@ -88,13 +90,14 @@ std::unique_ptr<Ring> new_ring(int device, size_t bytes)
     return nullptr;
 }
 
-// An idle ring of the device with room for bytes; else, if it may be allocated,
-// a new one in the place of a smaller idle one or within MAX_RINGS; else none.
+// An idle ring of the device with room for bytes; else, where allocate is not 0, a
+// new one of so many in the place of a smaller idle one or within MAX_RINGS; else
+// none.
 struct Lease {
     std::unique_ptr<Ring> ring;
     hipStream_t stream;
     bool done = false; // every copy into the ring has ended
-    Lease(int device, hipStream_t s, size_t bytes, bool allocate) : stream(s)
+    Lease(int device, hipStream_t s, size_t bytes, size_t allocate) : stream(s)
     {
         std::unique_ptr<Ring> drop;
         {
@@ -114,7 +117,7 @@ struct Lease {
         }
         drop.reset();
         try {
-            ring = new_ring(device, bytes);
+            ring = new_ring(device, allocate);
         } catch (const std::bad_alloc &) {
         }
         if (!ring) {
@@ -196,10 +199,12 @@ bool copy_to_host(Handle &h, const HostCopy *all, int n_all, const int *stop)
     const size_t piece = std::clamp((total / 4 + 4095) & ~size_t(4095), PIECE_MIN, SLOT_BYTES);
     std::unique_ptr<Lease> lease;
     if (n_items > 1 || total >= SINGLE_MIN) {
-        h.copied_to_host += total + size_t(n_items - 1) * RESULT_COST;
         const size_t pieces = padded / piece + 2; // the item that decides has its own
-        lease = std::make_unique<Lease>(h.device, h.stream, padded <= piece ? padded : std::min(pieces, size_t(SLOTS)) * piece,
-                                        h.copied_to_host >= RING_AFTER);
+        const size_t need = padded <= piece ? padded : std::min(pieces, size_t(SLOTS)) * piece;
+        h.host_ring = std::max(h.host_ring, std::bit_ceil(std::max(need, PIECE_MIN))); // few sizes: a ring is seldom replaced
+        const bool pays = std::max(h.copied_to_host, total) >= RING_PAYS * h.host_ring;
+        lease = std::make_unique<Lease>(h.device, h.stream, need, pays ? h.host_ring : 0);
+        h.copied_to_host += total + size_t(n_items - 1) * RESULT_COST;
     }
     if (!lease || !lease->ring) return copy_plain(h, all, n_all, stop);
     Ring &ring = *lease->ring;

@@ -131,8 +131,8 @@ bool plan_wave_gather(const Pattern &pat, int order, int n_quad, const int32_t *
 // E + G + H of 0.6 to 1.1 million P1 tets, wavefronts / the better row units, us:
 //   one point FP64: lattice (share 0.73) 175 / 200, BCC points moved by 5 %
 //   (0.68) 255 / 255, by 15 % (0.53) 292 / 259, by 25 % (0.30) 447 / 269, cubic
-//   lattice points by 30 % (0.23) 586 / 291; with large nodes 267 / 307 (0.65), 303 / 315 (0.53),
-//   460 / 331 (0.30), 604 / 381 (0.23)
+//   lattice points by 30 % (0.23) 586 / 291; with large nodes 267 / 307 (0.65),
+//   303 / 315 (0.53), 460 / 331 (0.30), 604 / 381 (0.23)
 //   one point FP32: lattice (0.93) 93 / 102, BCC 5 % (0.91) 129 / 128, 15 %
 //   (0.84) 130 / 131 and with another numbering 144 / 136, 25 % (0.79) 143 / 135;
 //   with large nodes 134 / 132 (0.91), 142 / 128 (0.84), 163 / 151 (0.81)

@@ -133,7 +133,7 @@ static const std::map<std::string, std::function<void()>> checks = {
     // arrays that DMA reaches are copied to once and directly, the others around them as ever
     {"pinned_destination", [] {
         Handle h;
-        copies(h, {4, 8 * MB, 100}, 4); // a handle in use
+        copies(h, {4, 8 * MB, 100}, 9); // a handle in use
         void *p = nullptr;
         const Bytes dev = data(9 * MB, 5), small = data(300 * KB, 6), flag(4, 0);
         (void)hipHostMalloc(&p, dev.size(), 0);
@@ -153,7 +153,7 @@ static const std::map<std::string, std::function<void()>> checks = {
     // all sizes around the limits
     {"sizes", [] {
         Handle h;
-        copies(h, {3 * MB, 3 * MB}, 6);
+        copies(h, {18 * MB, 3 * MB}, 5);
         for (size_t n : {size_t(1), size_t(16), 65 * KB, 1 * MB - 20, 1 * MB, 2 * MB - 1, 2 * MB, 4 * MB + 5, 17 * MB + 7}) {
             copies(h, {n}, 1);
             copies(h, {n, 5, n / 2 + 1}, 2);
@@ -167,8 +167,10 @@ static const std::map<std::string, std::function<void()>> checks = {
         Handle h;
         copies(h, {4, 8, 3000, 20 * KB}, 1);
         CHECK(most_queued == 1 && n_pageable == 4);
+        copies(h, {18 * MB}, 4);
+        CHECK(n_pageable == 8 && n_alloc == 0);
         copies(h, {18 * MB}, 1);
-        CHECK(n_pageable == 4);
+        CHECK(n_pageable == 8 && n_alloc == 1);
         for (size_t n : {8 * KB, 70 * KB, 300 * KB, 1 * MB}) {
             n_pageable = 0;
             copies(h, {4, n}, 1);
@@ -183,7 +185,7 @@ static const std::map<std::string, std::function<void()>> checks = {
     // flight, then the same ring under another handle
     {"kept_back", [] {
         Handle a, b;
-        copies(a, {20 * MB}, 3);
+        copies(a, {20 * MB}, 5);
         for (int k = 0; k < 4; ++k) {
             guarded(a, 1, (k % 2 ? 18 : 10) * MB);
             copies(b, {8, 300 * KB, 9 * MB}, 1);
@@ -196,6 +198,8 @@ static const std::map<std::string, std::function<void()>> checks = {
             copies(h, {8, 9 * MB}, 1);
             Handle g;
             copies(g, {8, 5000, 300 * KB}, 4);
+            Handle twice;
+            copies(twice, {20 * MB}, 2);
         }
         CHECK(n_alloc == 0);
     }},
@@ -214,7 +218,7 @@ static const std::map<std::string, std::function<void()>> checks = {
                 copies(g, {8, 20 * KB, 300 * KB}, 1);
                 CHECK(n_pageable == waits);
             }
-            copies(h, {18 * MB}, 3); // the ring is replaced
+            copies(h, {18 * MB}, 5); // the ring is replaced
             CHECK(n_alloc == 2 && n_free == 1 && largest <= 16 * MB);
         }
         CHECK(n_free == 2 && pinned.empty());
