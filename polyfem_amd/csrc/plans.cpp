@@ -261,10 +261,12 @@ bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, 
             for (int k = i; k < j; ++k) out.unused.push_back(k);
         }
         i = j;
+        // the share if the rest filled its chunks; in the end, the share
+        const double chunks = double(head.size()) + double(np[size_t(N)] - np[size_t(i)]) / cap;
+        out.share = chunks > 0 ? double(np[size_t(N)]) / (chunks * cap) : 1.0;
+        if (out.share < least_share) return false;
     }
     const int nc = int(head.size());
-    out.share = nc ? double(np[size_t(N)]) / (double(nc) * cap) : 1.0;
-    if (out.share < least_share) return false;
     std::vector<uint32_t> desc(static_cast<size_t>(nw), 0), long_desc(size_t(2 * nl));
     std::vector<uint16_t> dst(size_t(nc) * size_t(cap) * size_t(NB), 0);
     parallel_ranges(nc, [&](int c0, int c1) {

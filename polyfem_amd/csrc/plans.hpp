@@ -90,7 +90,7 @@ struct WavePlanHost {
 // an entry; word_limit: stage words of any chunk.  False when a row has more
 // than 64 rounds (at most 2) units, WAVE_BLOCKS blocks or 64 long blocks, its
 // stage exceeds word_limit or 64 KB, or the share is below least_share (found
-// before the lanes are dealt).
+// before the lanes are dealt, and as soon as the rows so far decide it).
 bool make_wave_plan(const Pattern &pat, int n_local, const int32_t *elem_nodes, int rounds, int word_cap,
                     int value_size, WavePlanHost &out, int word_limit = 16384, double least_share = 0);
 
